@@ -417,6 +417,15 @@ unsigned qsmi_fft_size(unsigned src) { return size_rule(src); }
 int qsmi_ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* fftSize, int nSub,
                    const float* subImages, qsmi_ti** out) {
   if (!out || !srcSize || !subImages) return fail(QSMI_ERR_ARG, "null argument");
+  return qsmi::ti_create(gpu, ndim, srcSize, fftSize, nSub, subImages, out);
+}
+
+}  // extern "C"
+
+namespace qsmi {
+
+int ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* fftSize, int nSub, const float* subImages,
+              qsmi_ti** out) {
   *out = nullptr;
   if (ndim < 1 || ndim > 3) return fail(QSMI_ERR_UNSUPPORTED, "ndim must be 1, 2 or 3");
   if (nSub < 1 || nSub > kMaxSub) return fail(QSMI_ERR_UNSUPPORTED, "nSub must be in [1, 16]");
@@ -486,6 +495,14 @@ int qsmi_ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* f
     }                                                                               \
   } while (0)
   TCHK(hipStreamCreateWithFlags(&t->stream, hipStreamNonBlocking));
+  // the 1024 x 1024 grid holds any 2-D TI of extents up to 1024 (valid
+  // positions never wrap); below grid1024Min the TI's own FFT grid is used
+  const int g1k = t->tune.grid1024Min;
+  t->w1k = (ndim == 2 && t->s[0] >= g1k && t->s[1] >= g1k && t->s[0] <= 1024 && t->s[1] <= 1024);
+  if (!subImages) {
+    *out = t;
+    return QSMI_OK;
+  }
   // twiddle tables, FP64-generated: tw[k] = exp(-2 pi i k / f)
   for (int i = 0; i < 3; ++i) {
     std::vector<float2> tw(t->f[i]);
@@ -535,10 +552,6 @@ int qsmi_ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* f
                   t->stream);
     TCHK(hipGetLastError());
   }
-  // the 1024 x 1024 grid holds any 2-D TI of extents up to 1024 (valid
-  // positions never wrap); below grid1024Min the TI's own FFT grid is used
-  const int g1k = t->tune.grid1024Min;
-  t->w1k = (ndim == 2 && t->s[0] >= g1k && t->s[1] >= g1k && t->s[0] <= 1024 && t->s[1] <= 1024);
   if (t->w1k) {
     std::vector<float2> tw(1024);
     std::vector<double2> twd(1024);
@@ -563,6 +576,10 @@ int qsmi_ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* f
   *out = t;
   return QSMI_OK;
 }
+
+}  // namespace qsmi
+
+extern "C" {
 
 int qsmi_ti_destroy(qsmi_ti* t) {
   if (!t) return QSMI_OK;
@@ -592,6 +609,7 @@ const TuneKey kTuneKeys[] = {
     {"fft.radix_max", &ScanTune::radixMax, 2, 13},
     {"fft.lognv_max", &ScanTune::lognvMax, 0, 6},
     {"loop.graph", &ScanTune::loopGraph, 0, 1},
+    {"loop.flow", &ScanTune::loopFlow, 0, 1},
 };
 const TuneKey* find_tune_key(const char* key) {
   if (!key) return nullptr;

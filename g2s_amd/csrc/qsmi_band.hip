@@ -481,9 +481,14 @@ size_t neighbour_lds(const ScanGeom& g, int nbMax) {
 
 bool exact_selection_on(const qsmi_device* dev) {
   if (dev->quantum != 0.f || dev->cross) return false;
-  const qsmi_ti* t = dev->ti;
   const int blocks = row_blocks(dev);
   return blocks <= kMaxBandBlocks;
+}
+
+bool exact_rows(const qsmi_ti* t) {
+  if (t->w1k) return true;
+  const long long rows = (long long)t->s[1] * t->s[2], per = 2 << t->lognv[0];
+  return (rows + per - 1) / per <= kMaxBandBlocks;
 }
 
 void band_free(BandBufs* b) {

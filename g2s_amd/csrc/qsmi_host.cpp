@@ -28,17 +28,16 @@
 #include <vector>
 
 #include "../../include/qsmi.h"
+#include "qsmi_flow.hpp"
 #include "qsmi_internal.hpp"
-
-namespace {
-
-}  // namespace
 
 extern "C" int qsmi_internal_fail(int code, const char* msg);
 
 namespace {
 
 int hfail(int code, const std::string& m) { return qsmi_internal_fail(code, m.c_str()); }
+
+int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow);
 
 struct KernelImg {
   int D = 0;
@@ -361,7 +360,84 @@ int qsmi_path(size_t cells, const unsigned char* informed, unsigned seed, unsign
 // ---------------------------------------------------------------------------
 // In-memory QS run
 // ---------------------------------------------------------------------------
-int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
+int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) { return qs_run(rq, rs, true); }
+
+}  // extern "C"
+
+namespace {
+
+// How the realisation qualifies for the data-flow path loop, or false. Its
+// direct form selects exactly as the exact selection does and its count form
+// as the tie quantum does when the quantum divides the weight, so only
+// requests whose wave loop would do the same qualify. tiIn, di: finite, and
+// small enough that no sum of squares overflows.
+bool plan_flow(const qsmi_qs_request* rq, const ScanTune& tune, int D, const float* tiIn, size_t S, size_t SD, int nMax,
+               const std::vector<int>& ncat, const std::vector<float>& catvals, const std::vector<float>& kernels,
+               int nExp, float quantum, qsmi::FlowPlan* F) {
+  const int nVar = rq->nVar;
+  if (!tune.loopFlow || tune.loopGraph || rq->nTI > 1 || rq->circularTI || rq->lp || rq->recordCap > 0 || rq->noVerbatim)
+    return false;
+  if (nVar > 8 || nExp > qsmi::kFlowMaxCat || (long long)nMax * nVar > qsmi::kFlowMaxTerms) return false;
+  if ((unsigned long long)S * nVar >= (1ull << 28) || SD >= (1ull << 31)) return false;
+  bool anyCat = false, anyCont = false;
+  int sub = 0, e = 0, ci = 0, cat = 0;
+  for (int v = 0; v < nVar; ++v) {
+    F->e0[v] = e;
+    if (rq->varTypes[v] == 0) {
+      anyCont = true;
+      sub += 2;
+      e += 1;
+    } else {
+      anyCat = true;
+      F->nCat[v] = ncat[ci];
+      F->cat0[v] = cat;
+      sub += ncat[ci];
+      e += ncat[ci];
+      cat += ncat[ci];
+      ++ci;
+    }
+  }
+  F->nClasses = cat;
+  const float w0 = kernels[0];
+  bool uniform = w0 > 0.f;
+  for (float w : kernels) {
+    if (!(w >= 0.f && w <= 1e6f)) return false;
+    uniform &= w == w0;
+  }
+  F->count = !anyCont && uniform;
+  F->mixed = anyCat;
+  if (F->count && quantum > 0.f) {
+    const float r = w0 / quantum;
+    if (!(r >= 2.f && r <= 65536.f && r == std::floor(r) && r * quantum == w0)) return false;
+  } else if (quantum != 0.f) {
+    return false;
+  }
+  // the exact selection's limit of its lists
+  if (quantum == 0.f && (size_t)nMax * (D * sizeof(int) + sub * sizeof(double)) + 8 > 48 * 1024) return false;
+  float big = 0.f;
+  for (size_t c = 0; c < S * nVar; ++c) big = std::max(big, std::fabs(tiIn[c]));
+  bool ok = big <= 1e12f;  // no TI value is NaN here
+  for (size_t c = 0; c < SD * nVar; ++c) ok &= !(std::fabs(rq->di[c]) > 1e12f);
+  if (!ok) return false;
+  F->unitW = uniform && w0 == 1.f;
+  // what the scan orders its terms by, from a sample of the TI
+  const size_t step = std::max<size_t>(1, S / 4096) | 1;
+  F->quant.assign((size_t)nVar * qsmi::kFlowQuant, 0.f);
+  for (int v = 0; v < nVar; ++v) {
+    std::vector<float> y;
+    for (size_t c = 0; c < S; c += step) y.push_back(tiIn[c * nVar + v]);
+    for (int q = 0; q < F->nCat[v]; ++q)
+      F->rare[F->cat0[v] + q] =
+          1.f - (float)std::count(y.begin(), y.end(), catvals[F->cat0[v] + q]) / (float)y.size();
+    if (rq->varTypes[v] != 0) continue;
+    std::sort(y.begin(), y.end());
+    for (int q = 0; q < qsmi::kFlowQuant; ++q)
+      F->quant[(size_t)v * qsmi::kFlowQuant + q] = y[(y.size() - 1) * (size_t)q / (qsmi::kFlowQuant - 1)];
+  }
+  return true;
+}
+
+int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   using clk = std::chrono::steady_clock;
   if (!rq || !rs || !rs->simulation || !rs->index) return hfail(QSMI_ERR_ARG, "null argument");
   const int D = rq->ndim;
@@ -582,21 +658,48 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
   unsigned begin = 0;
   qsmi_path(SD, informed.data(), rq->seed, path.data(), seeds.data(), &begin);
   const size_t nPath = SD - begin;
-  // device: TI spectra + scan engine
-  std::vector<float> sub((size_t)nSub * S);
-  if (cross)
-    qsmi_ti_subimages_x(D, s, nVar, rq->varTypes, tiData, sub.data());
-  else
-    qsmi_ti_subimages(D, s, nVar, rq->varTypes, tiIn, ncat.data(), catvals.data(), sub.data());
+  bool anyCont = false;
+  for (int v = 0; v < nVar; ++v) anyCont |= rq->varTypes[v] == 0;
+  float quantum = rq->tieQuantum;
+  if (quantum < 0.f) {
+    quantum = 0.f;
+    if (!anyCont && maxw > 0.f) {
+      int e2 = (int)std::ceil(std::log2((double)nMax * (double)maxw));
+      quantum = std::ldexp(1.f, e2 - 16);
+    }
+  }
+  // the data-flow path loop needs neither spectra nor a scan device
   qsmi_ti* ti = nullptr;
   qsmi_device* dev = nullptr;
-  int rc = qsmi_ti_create(rq->gpu, D, s, nullptr, nSub, sub.data(), &ti);
-  if (rc) return rc;
-  rc = qsmi_device_create(ti, alpha, rq->circularTI ? 1 : 0, &dev);
-  if (!rc && cross) rc = qsmi::set_cross(dev, alphaX, centreOk.data());
-  // the other TIs: spectra and a device each
+  qsmi::FlowPlan flow;
+  bool useFlow = allowFlow && !cross &&
+                 plan_flow(rq, qsmi::default_tune(), D, tiIn, S, SD, nMax, ncat, catvals, ker.data, nExp, quantum,
+                           &flow);
+  int rc = QSMI_OK;
+  if (useFlow) {
+    rc = qsmi::ti_create(rq->gpu, D, s, nullptr, nSub, nullptr, &ti);
+    if (rc) return rc;
+    if (quantum == 0.f && !qsmi::exact_rows(ti)) {  // the wave loop's FP32 selection
+      qsmi_ti_destroy(ti);
+      ti = nullptr;
+      useFlow = false;
+    }
+  }
+  // device: TI spectra + scan engine
   std::vector<qsmi_ti*> xti;
   std::vector<qsmi_device*> xdev;
+  if (!useFlow) {
+    std::vector<float> sub((size_t)nSub * S);
+    if (cross)
+      qsmi_ti_subimages_x(D, s, nVar, rq->varTypes, tiData, sub.data());
+    else
+      qsmi_ti_subimages(D, s, nVar, rq->varTypes, tiIn, ncat.data(), catvals.data(), sub.data());
+    rc = qsmi_ti_create(rq->gpu, D, s, nullptr, nSub, sub.data(), &ti);
+    if (rc) return rc;
+    rc = qsmi_device_create(ti, alpha, rq->circularTI ? 1 : 0, &dev);
+  }
+  if (!rc && cross) rc = qsmi::set_cross(dev, alphaX, centreOk.data());
+  // the other TIs: spectra and a device each
   for (int t = 1; t < nTI && !rc; ++t) {
     std::vector<float> subT((size_t)nSub * (cumT[t + 1] - cumT[t]));
     qsmi_ti_subimages(D, sT[t].data(), nVar, rq->varTypes, tiIn + cumT[t] * nVar, ncat.data(), catvals.data(),
@@ -620,17 +723,7 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
     qsmi_ti_destroy(ti);
     return rc;
   }
-  bool anyCont = false;
-  for (int v = 0; v < nVar; ++v) anyCont |= rq->varTypes[v] == 0;
-  float quantum = rq->tieQuantum;
-  if (quantum < 0.f) {
-    quantum = 0.f;
-    if (!anyCont && maxw > 0.f) {
-      int e2 = (int)std::ceil(std::log2((double)nMax * (double)maxw));
-      quantum = std::ldexp(1.f, e2 - 16);
-    }
-  }
-  qsmi_set_tie_quantum(dev, quantum);
+  if (dev) qsmi_set_tie_quantum(dev, quantum);
   for (qsmi_device* d : xdev) qsmi_set_tie_quantum(d, quantum);
   // output state
   float* di = rs->simulation;
@@ -653,6 +746,7 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
     *dst = p;
     return QSMI_OK;
   };
+  const hipStream_t stream = dev ? dev->stream : ti->stream;
   // path index of every cell, -1 for hard data (the posterior order of
   // src/qs.cpp:1615-1641: hard data first, then the path)
   const int n = nMax;
@@ -705,7 +799,7 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
   }
   if (!rc)
     rc = qsmi::nb_search_device(D, sd, nPath, (const unsigned*)dCells, (const int*)dPostS, (const int*)dOffs, nOff, n,
-                                (int*)dNb, (int*)dPj, (int*)dCnt, dev->stream, (const int*)dNNode,
+                                (int*)dNb, (int*)dPj, (int*)dCnt, stream, (const int*)dNNode,
                                 (const int*)dNodeKer, (const int*)dOffStart, (const int*)dOffCount,
                                 rq->circularSim ? 1 : 0);
   // learned proposal: which nodes reach the stencil coverage it needs
@@ -719,16 +813,16 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
                               (unsigned char*)dOk, dev->stream);
   }
   // dependency levels (1 + the deepest level among a node's path neighbours)
-  // on the device; only the levels come back
+  // on the device; only the levels come back (the data-flow loop waits for
+  // values instead and needs none)
   std::vector<int> level(nPath, 0);
   void *dLevel = nullptr, *dLvErr = nullptr;
   if (!rc) rc = dev_upload(nullptr, nPath * sizeof(int), &dLevel);
   if (!rc) rc = dev_upload(nullptr, sizeof(int), &dLvErr);
-  if (!rc) rc = qsmi::levels_device(nPath, n, (const int*)dPj, (const int*)dCnt, (int*)dLevel, (int*)dLvErr,
-                                    dev->stream);
+  if (!rc) rc = qsmi::levels_device(nPath, n, (const int*)dPj, (const int*)dCnt, (int*)dLevel, (int*)dLvErr, stream);
   int lvErr = 0;
   if (!rc) {
-    hipError_t e = hipStreamSynchronize(dev->stream);
+    hipError_t e = hipStreamSynchronize(stream);
     if (e == hipSuccess && nPath) e = hipMemcpy(level.data(), dLevel, nPath * sizeof(int), hipMemcpyDeviceToHost);
     if (e == hipSuccess) e = hipMemcpy(&lvErr, dLvErr, sizeof(int), hipMemcpyDeviceToHost);
     if (e == hipSuccess && dOk) {
@@ -753,15 +847,16 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
   }
   const auto tNb = clk::now();
   int maxLevel = 0;
-  for (size_t i = 0; i < nPath; ++i) maxLevel = std::max(maxLevel, level[i]);
+  const size_t nLeveled = level.size();
+  for (size_t i = 0; i < nLeveled; ++i) maxLevel = std::max(maxLevel, level[i]);
   // nodes ordered by (level, path order)
   std::vector<size_t> lvStart(maxLevel + 2, 0);
-  for (size_t i = 0; i < nPath; ++i) lvStart[level[i] + 1]++;
+  for (size_t i = 0; i < nLeveled; ++i) lvStart[level[i] + 1]++;
   for (int l = 0; l <= maxLevel; ++l) lvStart[l + 1] += lvStart[l];
-  std::vector<unsigned> order(nPath);
+  std::vector<unsigned> order(nLeveled);
   {
     std::vector<size_t> fillp(lvStart.begin(), lvStart.end() - 1);
-    for (size_t i = 0; i < nPath; ++i) order[fillp[level[i]]++] = (unsigned)i;
+    for (size_t i = 0; i < nLeveled; ++i) order[fillp[level[i]]++] = (unsigned)i;
   }
   // 512 nodes per wave measured best on the 1000x1000 path (fewer launches;
   // 768 no better); the learned proposal keeps its queries in LDS: 256
@@ -881,7 +976,24 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
     R.dPathK = (const float*)dPathK;
     R.dNodeKer = (const int*)dNodeKer;
     R.dNodeTi = (const int*)dNodeTi;
-    rc = qsmi::run_resident_waves(dev, R, stageMs, &scanned, &waves, bandStats);
+    if (useFlow) {
+      flow.nPath = (long long)nPath;
+      if (rq->waveSize > 0) {  // at most that many nodes at a time
+        flow.inFlight = rq->waveSize;
+        flow.segment = (int)std::min<long long>(flow.segment, 64ll * rq->waveSize);
+      }
+      bool gaveUp = false;
+      rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &gaveUp);
+      scanned = (long long)nPath;
+      waves = (int)R.waveLevel.size();
+      if (!rc && gaveUp) {  // a device wait hit its bound: the wave loop, from the start
+        for (void* p : allocs) (void)hipFree(p);
+        qsmi_ti_destroy(ti);
+        return qs_run(rq, rs, false);
+      }
+    } else {
+      rc = qsmi::run_resident_waves(dev, R, stageMs, &scanned, &waves, bandStats);
+    }
   }
   if (!rc) {
     hipError_t e = hipMemcpy(di, dDi, SD * nVar * sizeof(float), hipMemcpyDeviceToHost);
@@ -904,7 +1016,7 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
   rs->phaseMs[3] = std::chrono::duration<double, std::milli>(tLoop - tUp).count();
   const auto t2 = clk::now();
   destroy_extra();
-  qsmi_device_destroy(dev);
+  if (dev) qsmi_device_destroy(dev);
   qsmi_ti_destroy(ti);
   if (rc) {
     return rc;
@@ -930,4 +1042,4 @@ int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) {
   return QSMI_OK;
 }
 
-}  // extern "C"
+}  // namespace

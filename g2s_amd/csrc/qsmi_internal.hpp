@@ -26,6 +26,8 @@ struct ScanTune {
   int lognvMax = 6;        // at most 2^lognvMax transforms per own-grid FFT block (read at creation)
   int loopGraph = 0;       // 1: the path loop replays each wave's kernels as one captured HIP graph
                            // (1024-grid scans on two lanes)
+  int loopFlow = 1;        // 1: realisations that qualify run the data-flow path loop (qsmi_flow.hip); 0, or
+                           // loopGraph: waves of FFT scans
 };
 
 struct qsmi_ti {
@@ -183,6 +185,11 @@ double scan_cells(const qsmi_device* dev);
 float map_scale(const qsmi_device* dev);
 int rows_per_block(const qsmi_device* dev);
 int row_blocks(const qsmi_device* dev);
+// qsmi_ti_create; without sub-images the checks, the geometry and the stream
+// only (the data-flow path loop scans without spectra)
+bool exact_rows(const qsmi_ti* t);  // the exact selection tracks the rows grid of this TI
+int ti_create(int gpu, int ndim, const unsigned* srcSize, const unsigned* fftSize, int nSub, const float* subImages,
+              qsmi_ti** out);
 long long c_stride(const qsmi_device* dev);
 int grow_wave_bufs(qsmi_device* dev, WaveBufs* b, int nNodes, int total, int K);
 void free_wave_bufs(WaveBufs* b);

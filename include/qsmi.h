@@ -435,7 +435,8 @@ typedef struct {
   long long nodes;         /* out: simulated path nodes */
   long long scannedNodes;  /* out: nodes that went through the scan (the rest
                               drew from the marginal) */
-  int waves;               /* out: waves launched */
+  int waves;               /* out: waves of the path (dependency levels cut into at most waveSize
+                              nodes); the data-flow loop runs them without a launch each */
   double phaseMs[4];       /* out: path loop phases: neighbour search, dependency
                               levels and waves, uploads, device loop */
   long long lpProposed;    /* out: nodes served by the learned proposal */

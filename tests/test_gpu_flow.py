@@ -1,0 +1,116 @@
+"""The data-flow path loop (tuning key loop.flow) against the wave loop, the
+general path of the same realisation: identical bytes. The selection of both
+is exact (FP64 values by the device rule, or whole counts under a tie quantum
+that divides the weight), so no tolerance applies. The requests cover every
+form that the data-flow loop takes: 1-3 dimensions, extents around the tile
+and word edges (16, 32, 64), list lengths, weights, given and partially given
+cells, images of n and k, several kernels, wrapping grids and images whose
+best positions tie by the thousand."""
+import sys
+
+import numpy as np
+import pytest
+
+import g2s_amd
+
+pytestmark = pytest.mark.gpu
+
+
+def _field(dims, rng, kind):
+    a = rng.standard_normal(tuple(reversed(dims)))
+    for ax in range(a.ndim):
+        a = a + np.roll(a, 1, ax) + 0.5 * np.roll(a, 2, ax)
+    a = (a - a.mean()) / a.std()
+    if kind == "cont":
+        return np.exp(a).reshape(-1)
+    if kind == "flat":
+        return np.zeros(a.size)
+    if kind == "steps":  # few distinct values: many exact ties
+        return np.round(a).reshape(-1)
+    return np.digitize(a, np.quantile(a, np.arange(1, int(kind)) / int(kind))).astype(float).reshape(-1)
+
+
+def _both(*args, **kw):
+    out = []
+    try:
+        for flow in (1, 0):
+            g2s_amd.set_default_tuning("loop.flow", flow)
+            s, i, st = g2s_amd.qs(*args, stage_timing=True, **kw)
+            out.append((s.tobytes(), i.tobytes(), st))
+    finally:
+        g2s_amd.set_default_tuning("loop.flow", 1)
+    assert out[0][0] == out[1][0] and out[0][1] == out[1][1]
+    # the data-flow loop has no gather stage of its own
+    assert out[0][2]["gather_ms"] == 0.0 < out[1][2]["gather_ms"] and out[0][2]["waves"] == out[1][2]["waves"]
+    return out[0][2], out[1][2]
+
+
+CASES = [
+    # kinds per variable, image, grid, n, k, extra
+    (("cont",), (300,), (120,), 9, 1.5, {}),
+    (("cont",), (17, 5), (12, 9), 4, 1.0, {}),
+    (("cont",), (64, 63), (31, 17), 12, 2.0, dict(hard=0.1)),
+    (("cont",), (33, 129), (40, 13), 80, 3.0, dict(csim=True)),
+    (("cont",), (37, 18, 9), (11, 7, 6), 25, 1.5, dict(hard=0.05)),
+    (("cont",), (97, 65), (20, 20), 30, 16.0, dict(weights="distance")),
+    (("cont",), (81, 70), (24, 20), 20, 1.5, dict(weights=0.5, nimg=True, kimg=True)),
+    (("cont",), (60, 61), (20, 16), 14, 1.5, dict(kernels=True)),
+    (("flat",), (48, 40), (10, 8), 6, 2.0, {}),
+    (("steps",), (70, 52), (16, 16), 3, 1.5, {}),
+    (("cont", "cont"), (55, 44), (18, 14), 16, 1.5, dict(partial=True)),
+    (("cont", "3"), (66, 50), (20, 14), 18, 1.5, dict(hard=0.1, partial=True)),
+    (("3", "cont"), (50, 41), (14, 12), 10, 1.2, {}),
+    (("2",), (31, 20), (16, 13), 7, 1.0, {}),
+    (("2",), (97, 33), (25, 21), 50, 1.2, dict(hard=0.1, csim=True)),
+    (("4",), (65, 40), (20, 12), 150, 5.0, dict(weights=2.0)),
+    (("3",), (40, 33, 12), (10, 9, 7), 40, 1.5, dict(kimg=True)),
+    (("3",), (400,), (90,), 11, 1.5, {}),
+    (("2", "3"), (60, 45), (15, 14), 20, 16.0, dict(partial=True, quantum=0.0)),
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_flow_equals_waves(case):
+    kinds, dims, sdims, n, k, x = CASES[case]
+    print(f"data-flow loop: case {case} {CASES[case]}", flush=True)
+    sys.stdout.flush()
+    rng = np.random.default_rng(100 + case)
+    types = [0 if q in ("cont", "flat", "steps") else 1 for q in kinds]
+    ti = np.stack([_field(dims, rng, q) for q in kinds], 1).astype(np.float32)
+    cells = int(np.prod(sdims))
+    di = np.full((cells, len(kinds)), np.nan, np.float32)
+    u = rng.random(cells)
+    src = ti[rng.integers(0, ti.shape[0], cells)]
+    if "hard" in x:
+        di[u < x["hard"]] = src[u < x["hard"]]
+    if "partial" in x:
+        one = u > 0.8
+        di[one, case % len(kinds)] = src[one, case % len(kinds)]
+    kd = [d // 2 + 1 for d in dims]
+    kw = dict(circular_sim=x.get("csim", False), tie_quantum=x.get("quantum", -1.0))
+    if "weights" in x:
+        if x["weights"] == "distance":
+            ker = g2s_amd.kernel_generate(kd, [2] * len(kinds), [1.0] * len(kinds), [0.05] * len(kinds))
+        else:
+            ker = np.full(int(np.prod(kd)) * len(kinds), x["weights"], np.float32)
+        kw.update(kernel=ker, kernel_dims=kd)
+    if "nimg" in x:
+        kw["n_image"] = rng.integers(0, n + 1, cells).astype(np.float32)
+    if "kimg" in x:
+        kw["k_image"] = rng.choice([1.0, k, 2.5], cells).astype(np.float32)
+    if "kernels" in x:
+        sizes = [kd, [9, 11]]
+        kw.update(kernels=[np.ones(int(np.prod(s)), np.float32) for s in sizes], kernels_dims=sizes,
+                  kernel_index_image=rng.integers(0, 2, cells).astype(np.float32))
+    _both(ti, dims, di, sdims, types, n, k, 5 + case, **kw)
+
+
+def test_flow_slices_and_segments():
+    """An image large enough for several slices a node and a path of several
+    launches (64 nodes in flight, 64 x 64 a launch)."""
+    rng = np.random.default_rng(3)
+    dims, sdims = (410, 390), (80, 70)
+    ti = _field(dims, rng, "cont").astype(np.float32)
+    di = np.full(int(np.prod(sdims)), np.nan, np.float32)
+    flow, waves = _both(ti, dims, di, sdims, [0], 24, 1.5, 4, wave_size=64)
+    assert flow["exact_nodes"] == waves["exact_nodes"]
