@@ -297,44 +297,49 @@ int qsmi_offsets(int ndim, const unsigned* ks, int kNVar, const float* kernel, i
   if (!ks || !out || !count || ndim < 1 || ndim > 3) return hfail(QSMI_ERR_ARG, "invalid argument");
   // generation order of src/qs.cpp:1055-1084: dimension by dimension, each
   // existing offset followed by its +j then -j copies
-  std::vector<std::vector<int>> list(1);
+  struct Off {
+    float key;  // -|d|^2
+    int d[3];
+  };
+  size_t total = 1;
+  for (int i = 0; i < ndim; ++i) total *= (size_t)(2 * (((int)ks[i] + 1) / 2) - 1);
+  std::vector<Off> list(total);
+  list[0] = Off{0.f, {0, 0, 0}};
+  size_t base = 1;
   for (int i = 0; i < ndim; ++i) {
-    const size_t base = list.size();
     const int half = ((int)ks[i] + 1) / 2;
-    for (auto& v : list) v.push_back(0);
-    list.resize(base * (size_t)(2 * half - 1));
     for (int j = 1; j < half; ++j) {
+      Off* pos = list.data() + base * (size_t)(2 * j - 1);
+      Off* neg = list.data() + base * (size_t)(2 * j);
       for (size_t q = 0; q < base; ++q) {
-        std::vector<int> a = list[q], b = list[q];
-        a[i] = j;
-        b[i] = -j;
-        list[base * (size_t)(2 * j - 1) + q] = a;
-        list[base * (size_t)(2 * j) + q] = b;
+        pos[q] = neg[q] = list[q];
+        pos[q].d[i] = j;
+        neg[q].d[i] = -j;
       }
     }
+    base *= (size_t)(2 * half - 1);
   }
   if (kernel) {  // NaN kernel weights remove the offset (centre (size-1)/2)
-    std::vector<std::vector<int>> kept;
-    kept.reserve(list.size());
-    for (auto& v : list) {
+    size_t kept = 0;
+    for (const Off& v : list) {
       size_t idx = 0;
       for (int i = ndim - 1; i >= 0; --i) {
-        int c = ((int)ks[i] - 1) / 2 + v[i];
+        int c = ((int)ks[i] - 1) / 2 + v.d[i];
         c = ((c % (int)ks[i]) + (int)ks[i]) % (int)ks[i];
         idx = idx * ks[i] + (size_t)c;
       }
-      if (!std::isnan(kernel[idx * kNVar])) kept.push_back(v);
+      if (!std::isnan(kernel[idx * kNVar])) list[kept++] = v;
     }
-    list.swap(kept);
+    list.resize(kept);
   }
   // the reference compares -|d|^2 with '>'; the same comparisons in the same
-  // libstdc++ introsort give the same order of equal-distance offsets
-  std::sort(list.begin(), list.end(), [&](const std::vector<int>& a, const std::vector<int>& b) {
-    return -dist2_center(ndim, ks, a.data()) > -dist2_center(ndim, ks, b.data());
-  });
+  // libstdc++ introsort give the same order of equal-distance offsets (the
+  // keys computed once: the order depends on the comparisons only)
+  for (Off& v : list) v.key = -dist2_center(ndim, ks, v.d);
+  std::sort(list.begin(), list.end(), [](const Off& x, const Off& y) { return x.key > y.key; });
   if ((int)list.size() > capacity) return hfail(QSMI_ERR_ARG, "offset capacity too small");
   for (size_t q = 0; q < list.size(); ++q)
-    for (int i = 0; i < ndim; ++i) out[q * ndim + i] = list[q][i];
+    for (int i = 0; i < ndim; ++i) out[q * ndim + i] = list[q].d[i];
   *count = (int)list.size();
   return QSMI_OK;
 }
