@@ -63,7 +63,7 @@ constexpr int SLOT_W = 2 * SLOT_R + 1;     // 17 x 17 map: canonical slot or -1
 constexpr int NSEG = 16;  // shortlist segments per node (one counter each)
 
 constexpr int GT = 64;   // block tile (M and N)
-constexpr int GK = 32;   // K step
+constexpr int GK = 128;  // K step
 constexpr int LDT = GK + 8;  // LDS row stride (bf16), 16-byte aligned fragments
 
 // ---------------------------------------------------------------------------
@@ -73,7 +73,16 @@ constexpr int LDT = GK + 8;  // LDS row stride (bf16), 16-byte aligned fragments
 // Epilogue EPI_STORE: C = (acc ? C : 0) + AB (+ bias[n]) (ReLU when relu);
 //          EPI_SELECT: positions n with AB[m][n] >= thr[m] are appended to
 //          list[m][...] (counter cnt[m], capacity cap; overflow only counts).
-// 256 threads: four wavefronts, each a 32 x 32 quarter of the 64 x 64 tile.
+//          Each value is zeroed where mask[m][n] <= 0 (the ReLU's backward).
+// 4 KW wavefronts: a 32 x 32 quarter of the 64 x 64 tile and, for KW = 4, a
+// quarter of every K step each, summed through LDS at the end.
+// These products are latency-bound (16 to 64 blocks): with a K step of 32 the
+// chain of load, store, barrier, product ran 32 times for a weight gradient
+// over 1024 rows (44 us); steps of 128 with the next step's loads issued before
+// the products run it 8 times. KW = 1 adds in K order, the order of the
+// encoders' values everywhere; the gradients take KW = 4. Each operand is read
+// along its contiguous dimension by neighbouring lanes and stored as 16-byte
+// runs of K.
 // ---------------------------------------------------------------------------
 enum { EPI_STORE = 0, EPI_SELECT = 1 };
 
@@ -88,6 +97,7 @@ struct GemmArgs {
   int accumulate;
   const float* bias;
   int relu;
+  const float* mask;  // row stride ldc
   // select epilogue
   const float* thr;
   uint32_t* list;
@@ -95,66 +105,100 @@ struct GemmArgs {
   int cap;
 };
 
-template <bool TA, bool TB, int EPI>
-__global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
-  __shared__ __attribute__((aligned(16))) __bf16 As[GT * LDT];
-  __shared__ __attribute__((aligned(16))) __bf16 Bs[GT * LDT];
+// Eight K-consecutive elements of one row of a tile. TR: K is the slow
+// dimension in memory (P[k][row]); rows / K past the edge are zero.
+template <bool TR>
+__device__ __forceinline__ void gemm_load(const float* __restrict__ P, int ld, int row, int rows, int k, int K,
+                                          float (&v)[8]) {
+  if (!TR && row < rows && k + 8 <= K && (ld & 3) == 0 && ((uintptr_t)P & 15) == 0) {
+    const float4* q = reinterpret_cast<const float4*>(P + (long long)row * ld + k);  // k is a multiple of 8
+    const float4 a = q[0], b = q[1];
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+    v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const bool in = row < rows && k + e < K;
+    v[e] = in ? (TR ? P[(long long)(k + e) * ld + row] : P[(long long)row * ld + k + e]) : 0.f;
+  }
+}
+
+__device__ __forceinline__ void gemm_put(__bf16* dst, const float (&v)[8]) {
+  bf16x8 x;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = (__bf16)v[e];
+  *reinterpret_cast<bf16x8*>(dst) = x;
+}
+
+template <bool TA, bool TB, int EPI, int KW>
+__global__ void __launch_bounds__(256 * KW) k_gemm(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) __bf16 sm[2 * GT * LDT];
+  __bf16 *As = sm, *Bs = sm + GT * LDT;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int quad = wave & 3, kw = wave >> 2;
   const int bm = blockIdx.y * GT, bn = blockIdx.x * GT;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+  const int wm = (quad >> 1) * 32, wn = (quad & 1) * 32;
+  // this thread's runs of each tile: lanes run along the operand's contiguous
+  // dimension
+  constexpr int RUNS = 4 / KW, THR = 256 * KW;
+  auto runOf = [&](bool tr, int j, int& row, int& k) {
+    const int t = tid + j * THR;
+    row = tr ? (t & 63) : (t >> 4);
+    k = (tr ? (t >> 6) : (t & 15)) * 8;
+  };
   f32x16 acc;
 #pragma unroll
   for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  for (int k0 = 0; k0 < g.K; k0 += GK) {
-    // A tile -> As[m][k]
-    if (!TA) {
-      const int m = tid >> 2, kb = (tid & 3) * 8;
-      const int gm = bm + m;
+  float va[RUNS][8], vb[RUNS][8];
+  auto load = [&](int k0) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int gk = k0 + kb + e;
-        const float v = (gm < g.M && gk < g.K) ? g.A[(long long)gm * g.lda + gk] : 0.f;
-        As[m * LDT + kb + e] = (__bf16)v;
-      }
-    } else {
-      const int k = tid >> 3, mb = (tid & 7) * 8;
-      const int gk = k0 + k;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int gm = bm + mb + e;
-        const float v = (gm < g.M && gk < g.K) ? g.A[(long long)gk * g.lda + gm] : 0.f;
-        As[(mb + e) * LDT + k] = (__bf16)v;
-      }
+    for (int j = 0; j < RUNS; ++j) {
+      int row, k;
+      runOf(TA, j, row, k);
+      gemm_load<TA>(g.A, g.lda, bm + row, g.M, k0 + k, g.K, va[j]);
+      runOf(!TB, j, row, k);
+      gemm_load<!TB>(g.B, g.ldb, bn + row, g.N, k0 + k, g.K, vb[j]);
     }
-    // B tile -> Bs[n][k]
-    if (TB) {
-      const int n = tid >> 2, kb = (tid & 3) * 8;
-      const int gn = bn + n;
+  };
+  load(0);
+  for (int k0 = 0; k0 < g.K; k0 += GK) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int gk = k0 + kb + e;
-        const float v = (gn < g.N && gk < g.K) ? g.B[(long long)gn * g.ldb + gk] : 0.f;
-        Bs[n * LDT + kb + e] = (__bf16)v;
-      }
-    } else {
-      const int k = tid >> 3, nb = (tid & 7) * 8;
-      const int gk = k0 + k;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int gn = bn + nb + e;
-        const float v = (gn < g.N && gk < g.K) ? g.B[(long long)gk * g.ldb + gn] : 0.f;
-        Bs[(nb + e) * LDT + k] = (__bf16)v;
-      }
+    for (int j = 0; j < RUNS; ++j) {
+      int row, k;
+      runOf(TA, j, row, k);
+      gemm_put(As + row * LDT + k, va[j]);
+      runOf(!TB, j, row, k);
+      gemm_put(Bs + row * LDT + k, vb[j]);
     }
     __syncthreads();
+    if (k0 + GK < g.K) load(k0 + GK);
 #pragma unroll
-    for (int s = 0; s < GK / 16; ++s) {
-      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&As[(wm + (lane & 31)) * LDT + 16 * s + 8 * (lane >> 5)]);
-      const bf16x8 b = *reinterpret_cast<const bf16x8*>(&Bs[(wn + (lane & 31)) * LDT + 16 * s + 8 * (lane >> 5)]);
+    for (int s = 0; s < 8 / KW; ++s) {
+      const int kk = (GK / KW) * kw + 16 * s + 8 * (lane >> 5);
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&As[(wm + (lane & 31)) * LDT + kk]);
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(&Bs[(wn + (lane & 31)) * LDT + kk]);
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
     }
     __syncthreads();
   }
+  // the K quarters of each 32 x 32 quarter tile: (2, 3) onto (0, 1), 1 onto 0
+  float* red = reinterpret_cast<float*>(sm);  // [2][4][16][64]
+  static_assert(sizeof(sm) >= 2 * 4 * 1024 * sizeof(float), "reduction space");
+#pragma unroll
+  for (int half = KW / 2; half >= 1; half >>= 1) {
+    if (kw >= half && kw < 2 * half) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) red[(((kw - half) * 4 + quad) * 16 + r) * 64 + lane] = acc[r];
+    }
+    __syncthreads();
+    if (kw < half) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[r] += red[((kw * 4 + quad) * 16 + r) * 64 + lane];
+    }
+    __syncthreads();
+  }
+  if (kw != 0) return;
   const int gn = bn + wn + (lane & 31);
 #pragma unroll
   for (int r = 0; r < 16; ++r) {
@@ -166,6 +210,7 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
       if (g.accumulate) v += *c;
       if (g.bias) v += g.bias[gn];
       if (g.relu) v = fmaxf(v, 0.f);
+      if (g.mask && !(g.mask[(long long)gm * g.ldc + gn] > 0.f)) v = 0.f;
       *c = v;
     } else {
       if (v >= g.thr[gm]) {
@@ -176,17 +221,23 @@ __global__ void __launch_bounds__(256) k_gemm(GemmArgs g) {
   }
 }
 
-void gemm(bool ta, bool tb, const GemmArgs& a, hipStream_t st) {
-  dim3 grid((a.N + GT - 1) / GT, (a.M + GT - 1) / GT);
-  if (!ta && !tb) hipLaunchKernelGGL((k_gemm<false, false, EPI_STORE>), grid, dim3(256), 0, st, a);
-  else if (!ta && tb) hipLaunchKernelGGL((k_gemm<false, true, EPI_STORE>), grid, dim3(256), 0, st, a);
-  else if (ta && !tb) hipLaunchKernelGGL((k_gemm<true, false, EPI_STORE>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((k_gemm<true, true, EPI_STORE>), grid, dim3(256), 0, st, a);
+template <int KW>
+void gemm_kw(bool ta, bool tb, const GemmArgs& a, hipStream_t st) {
+  dim3 grid((a.N + GT - 1) / GT, (a.M + GT - 1) / GT), block(256 * KW);
+  if (!ta && !tb) hipLaunchKernelGGL((k_gemm<false, false, EPI_STORE, KW>), grid, block, 0, st, a);
+  else if (!ta && tb) hipLaunchKernelGGL((k_gemm<false, true, EPI_STORE, KW>), grid, block, 0, st, a);
+  else if (ta && !tb) hipLaunchKernelGGL((k_gemm<true, false, EPI_STORE, KW>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_gemm<true, true, EPI_STORE, KW>), grid, block, 0, st, a);
 }
+
+void gemm(bool ta, bool tb, const GemmArgs& a, hipStream_t st) { gemm_kw<1>(ta, tb, a, st); }
+
+// the products of the backward pass
+void gemm_grad(bool ta, bool tb, const GemmArgs& a, hipStream_t st) { gemm_kw<4>(ta, tb, a, st); }
 
 void gemm_select(const GemmArgs& a, hipStream_t st) {
   dim3 grid((a.N + GT - 1) / GT, (a.M + GT - 1) / GT);
-  hipLaunchKernelGGL((k_gemm<false, true, EPI_SELECT>), grid, dim3(256), 0, st, a);
+  hipLaunchKernelGGL((k_gemm<false, true, EPI_SELECT, 1>), grid, dim3(256), 0, st, a);
 }
 
 GemmArgs gargs(int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc) {
@@ -207,19 +258,26 @@ GemmArgs gargs(int M, int N, int K, const float* A, int lda, const float* B, int
 // ---------------------------------------------------------------------------
 // element-wise kernels
 // ---------------------------------------------------------------------------
-// dY *= (Y > 0) (ReLU backward, Y = the layer's output after ReLU)
-__global__ void k_relu_bwd(float* __restrict__ dy, const float* __restrict__ y, long long n) {
-  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n && !(y[i] > 0.f)) dy[i] = 0.f;
-}
-
-// db[n] (+)= sum_r dY[r][n]
-__global__ void k_colsum(const float* __restrict__ dy, int rows, int cols, float* __restrict__ db) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
+// db[n] = sum_r dY[r][n]: eight columns a block, 32 threads a column, each
+// summing every 32nd row, then the 32 sums in a fixed order (one thread a
+// column took 141 us for 1024 rows: a chain of 1024 dependent loads and adds)
+__global__ void __launch_bounds__(256) k_colsum(const float* __restrict__ dy, int rows, int cols,
+                                                float* __restrict__ db) {
+  __shared__ float part[32][9];
+  const int c = threadIdx.x & 7, g = threadIdx.x >> 3, col = blockIdx.x * 8 + c;
   float s = 0.f;
-  for (int r = 0; r < rows; ++r) s += dy[(long long)r * cols + c];
-  db[c] = s;
+  if (col < cols) {
+#pragma unroll 8
+    for (int r = g; r < rows; r += 32) s += dy[(long long)r * cols + col];
+  }
+  part[g][c] = s;
+  __syncthreads();
+  if (g == 0 && col < cols) {
+    float t = 0.f;
+#pragma unroll
+    for (int q = 0; q < 32; ++q) t += part[q][c];
+    db[col] = t;
+  }
 }
 
 // Softmax cross-entropy of row b of G * invTau against column b (one block
@@ -937,16 +995,14 @@ void backward(qsmi_lp* lp, int t, const Acts& a, float* dE, int n, float* dHa, f
   float* dOut = dE;
   for (int l = 3; l >= 0; --l) {
     const float* in = l > 0 ? a.H[l - 1] : a.X;
-    gemm(true, false, gargs(kDin[l], kDout[l], n, in, kDin[l], dOut, kDout[l], G + kWoff[l], kDout[l]), lp->stream);
-    hipLaunchKernelGGL(k_colsum, dim3((kDout[l] + 255) / 256), dim3(256), 0, lp->stream, dOut, n, kDout[l],
+    gemm_grad(true, false, gargs(kDin[l], kDout[l], n, in, kDin[l], dOut, kDout[l], G + kWoff[l], kDout[l]), lp->stream);
+    hipLaunchKernelGGL(k_colsum, dim3((kDout[l] + 7) / 8), dim3(256), 0, lp->stream, dOut, n, kDout[l],
                        G + boff(l));
     if (l > 0) {
       float* dIn = (l & 1) ? dHa : dHb;
-      gemm(false, true, gargs(n, kDin[l], kDout[l], dOut, kDout[l], W + kWoff[l], kDout[l], dIn, kDin[l]),
-           lp->stream);
-      const long long cnt = (long long)n * kDin[l];
-      hipLaunchKernelGGL(k_relu_bwd, dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, lp->stream, dIn, a.H[l - 1],
-                         cnt);
+      GemmArgs g = gargs(n, kDin[l], kDout[l], dOut, kDout[l], W + kWoff[l], kDout[l], dIn, kDin[l]);
+      g.mask = a.H[l - 1];
+      gemm_grad(false, true, g, lp->stream);
       dOut = dIn;
     }
   }
@@ -971,8 +1027,8 @@ void loss_backward(qsmi_lp* lp, const Acts& q, const Acts& k, const LossBufs& L,
   hipStream_t st = lp->stream;
   gemm(false, true, gargs(B, C, EMB, q.E, EMB, k.E, EMB, L.Gm, C), st);
   hipLaunchKernelGGL(k_softmax_ce, dim3(B), dim3(256), 0, st, L.Gm, B, C, invTau, L.dG, L.loss);
-  gemm(false, false, gargs(B, EMB, C, L.dG, C, k.E, EMB, L.dQ, EMB), st);
-  gemm(true, false, gargs(C, EMB, B, L.dG, C, q.E, EMB, L.dK, EMB), st);
+  gemm_grad(false, false, gargs(B, EMB, C, L.dG, C, k.E, EMB, L.dQ, EMB), st);
+  gemm_grad(true, false, gargs(C, EMB, B, L.dG, C, q.E, EMB, L.dK, EMB), st);
   backward(lp, 0, q, L.dQ, B, L.dHa, L.dHb);
   backward(lp, 1, k, L.dK, C, L.dHa, L.dHb);
 }
