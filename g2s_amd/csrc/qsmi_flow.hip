@@ -179,6 +179,9 @@ struct FlowShared {
   float thr;
   uint32_t bound;  // smallest K-th cost a wavefront of the block knows
   int unit;        // units handed out
+  int flushed;     // a wavefront has scored positions before the end
+  uint32_t few[16];  // the positions left at the end of a slice, and their values
+  double fewVal[16];
   float delta0;
   uint32_t pos[kMaxK];
 };
@@ -259,18 +262,23 @@ __device__ __forceinline__ void gather_node(FlowArgs& P, int i, unsigned cell, i
 #pragma unroll
     for (int v = 0; v < NV; ++v)
       if (v < P.nVar) bits[v] = ld_agent(&wp[v]);
+    // the position the neighbour was copied from, moved back by its offset
+    // (hard data and stale entries give 0: any position may seed the bound)
+    unsigned sp = ld_agent(&P.index[t]);
+    bool waited = false;
     float val[NV];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
       if (v >= P.nVar) continue;
       uint32_t b = bits[v];
-      if (b == kPending && t != cell) b = wait_word(&wp[v], &P.ctl[1]);
+      if (b == kPending && t != cell) {
+        b = wait_word(&wp[v], &P.ctl[1]);
+        waited = true;
+      }
       val[v] = (b == kPending || b == kEmpty) ? NAN : __uint_as_float(b);
     }
     if (j >= 1 && j <= kSources) {
-      // the position the neighbour was copied from, moved back by its offset
-      // (hard data and stale entries give 0: any position may seed the bound)
-      const unsigned sp = ld_agent(&P.index[t]);
+      if (waited) sp = ld_agent(&P.index[t]);
       sh->src[j - 1][0] = (int)(sp % (unsigned)P.s[0]) - dd[0];
       sh->src[j - 1][1] = (int)((sp / (unsigned)P.s[0]) % (unsigned)P.s[1]) - dd[1];
       sh->src[j - 1][2] = (int)(sp / ((unsigned)P.s[0] * (unsigned)P.s[1])) - dd[2];
@@ -557,6 +565,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
   nb.dt = nb.w + nv;
   nb.d0 = reinterpret_cast<int*>(nb.dt + nv);
   nb.row = nb.d0 + P0.n;
+  __builtin_amdgcn_s_setprio(3);
   for (int t = tid; t < nVar * kFlowQuant; t += kThreads) quant[t] = P0.quant[t];  // first read after a barrier
   unsigned long long nScored = 0, nNodesDone = 0, nFlush = 0;
   for (;;) {
@@ -663,6 +672,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
       float c = 0.f;
       if (sp != kNone) {
         const char* b = pl + (size_t)sp * 4;
+#pragma unroll 4
         for (int t = sub; t < Tn; t += 8) {
           const float d = *reinterpret_cast<const float*>(b + tOff[t]) - tX[t];
           float d2 = d * d;
@@ -677,6 +687,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
         sh.thr = INFINITY;
         sh.bound = 0x7F800000u;
         sh.unit = 0;
+        sh.flushed = 0;
       }
       __syncthreads();
       if (tid < kSources) {
@@ -700,6 +711,9 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
     tk.init();
     const int NX = (n[0] + kTileX * kPair - 1) / (kTileX * kPair), NY = (n[1] + kTileY - 1) / kTileY;
     const int units = box ? NX * NY * n[2] : 0;
+    // a node's dependents wait for everything but the scan's share of the
+    // other nodes: the scan yields to the short phases around it
+    __builtin_amdgcn_s_setprio(0);
     if (slice * kRun < units) {
       const int lx = lane & (kTileX - 1), ly = lane / kTileX;
       const uint32_t laneVo = (uint32_t)(lx + s0 * ly) * 4u;
@@ -814,6 +828,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           nScored += score_list<NV, KT>(P, nb, cnt, delta0, seedbits, lPos[wave], lCost[wave], len, lim, lane, tk);
           ++nFlush;
+          sh.flushed = 1;
           len = 0;
         }
         // what the other wavefronts of the block know
@@ -824,12 +839,63 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
         }
       }
     }
+    __builtin_amdgcn_s_setprio(3);
     // the slice's bound: every wavefront's K-th cost holds for all
     if (lane == 0) sh.f[wave] = thr;
     __syncthreads();
     lim = cost_limit(fminf(fminf(sh.f[0], sh.f[1]), fminf(sh.f[2], sh.f[3])), W, Tn);
-    nScored += score_list<NV, KT>(P, nb, cnt, delta0, seedbits, lPos[wave], lCost[wave], len, lim, lane, tk);
-    block_topk64<KT>(tk, K, best, red);
+    // few positions are left as a rule: into one list, scored by all wavefronts
+    int kept = 0;
+    for (int e = lane; e < len; e += 64) kept += lCost[wave][e] <= lim ? 1 : 0;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) kept += __shfl_xor(kept, off);
+    if (lane == 0) sh.m[wave] = kept;
+    __syncthreads();
+    const int total = __builtin_amdgcn_readfirstlane(sh.m[0] + sh.m[1] + sh.m[2] + sh.m[3]);
+    const bool flushed = __builtin_amdgcn_readfirstlane(sh.flushed) != 0;
+    if (total <= 16 && !flushed && NV <= 2) {  // block-uniform
+      int at = 0;
+      for (int w = 0; w < wave; ++w) at += sh.m[w];
+      for (int e0 = 0; e0 < len; e0 += 64) {
+        const int e = e0 + lane;
+        const bool ok = e < len && lCost[wave][e] <= lim;
+        const unsigned long long m = __ballot(ok);
+        if (ok) sh.few[at + __popcll(m & ((1ull << lane) - 1ull))] = lPos[wave][e];
+        at += __popcll(m);
+      }
+      __syncthreads();
+      for (int e = wave; e < total; e += kWaves) {
+        const double v = exact_wave<NV>(P, nb, cnt, delta0, __builtin_amdgcn_readfirstlane(sh.few[e]), lane);
+        if (lane == 0) sh.fewVal[e] = v;
+      }
+      nScored += wave == 0 ? total : 0;
+      __syncthreads();
+      if (tid < 64) {  // rank of each among all
+        Cand64 c = worst_cand64();
+        if (lane < total) {
+          c.val = sh.fewVal[lane];
+          c.pos = sh.few[lane];
+          c.h = tie_hash(seedbits, c.pos);
+        }
+        int rank = 0;
+        for (int e = 0; e < total; ++e) {
+          Cand64 o;
+          o.val = readlane64(c.val, e);
+          o.h = (uint32_t)__builtin_amdgcn_readlane((int)c.h, e);
+          o.pos = (uint32_t)__builtin_amdgcn_readlane((int)c.pos, e);
+          rank += cand64_better(o, c) ? 1 : 0;
+        }
+        if (lane < total) {
+          if (rank < K) best[rank] = c;
+        } else if (lane < K) {
+          best[lane] = c;
+        }
+      }
+      __syncthreads();
+    } else {
+      nScored += score_list<NV, KT>(P, nb, cnt, delta0, seedbits, lPos[wave], lCost[wave], len, lim, lane, tk);
+      block_topk64<KT>(tk, K, best, red);
+    }
     if (G > 1) {
       unsigned long long* sl = P.slots + (long long)q * (G - 1) * K * 2;
       if (slice < G - 1) {
@@ -880,6 +946,7 @@ struct BitTerms {
 __device__ __forceinline__ int count_at(const char* bits, const BitTerms& bt, int T, int c0, uint32_t rb, int t0,
                                         int step) {
   int c = 0;
+#pragma unroll 4
   for (int t = t0; t < T; t += step) {
     const int b = c0 + bt.sh[t];
     const uint32_t w = *reinterpret_cast<const uint32_t*>(bits + bt.off[t] + rb + (uint32_t)(b >> 5) * 4u);
@@ -998,6 +1065,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
       br[k] = 0ull;
       bp[k] = kNone;
     }
+    __builtin_amdgcn_s_setprio(0);
     // every G-th run of 64 units belongs to the slice, handed out to its wavefronts
     for (;;) {
       int k = 0;
@@ -1107,6 +1175,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
       // what the other wavefronts of the block know
       thr = __builtin_amdgcn_readfirstlane(max(thr, *(volatile int*)&sh.m[0]));
     }
+    __builtin_amdgcn_s_setprio(3);
     // K rounds of block maxima
     auto block_best = [&]() {
       for (int k = 0; k < K; ++k) {
@@ -1245,7 +1314,7 @@ hipError_t launch_persistent(F kernel, const FlowParams& P, size_t lds, int maxB
 // idle where few nodes are independent.
 static int flow_slices(const FlowPlan& F, long long S, int terms) {
   const long long pairs = S * terms;
-  const long long per = F.count ? 4000000 : 160000;
+  const long long per = F.count ? 1000000 : 160000;
   return (int)std::max<long long>(1, std::min<long long>(48, pairs / per));
 }
 

@@ -387,33 +387,42 @@ __global__ void __launch_bounds__(64) k_nbsearch(int D, int sd0, int sd1, int sd
   const int o0 = nodeKer ? offStart[nodeKer[i]] : 0;
   const int nO = nodeKer ? offCount[nodeKer[i]] : nOff;
   int cnt = 0;
-  for (int base = 0; base < nO && cnt < nI; base += 64) {
-    const int o = o0 + base + lane;
-    bool hit = false;
-    int pj = -1;
-    if (base + lane < nO) {
-      bool inside = true;
-      long long t = 0, mul = 1;
+  // kSearch rounds of 64 offsets at a time: the loads of all rounds are in
+  // flight together (the first nodes of a path walk the whole list: 4.6 ms for
+  // 416,325 offsets one round at a time)
+  constexpr int kSearch = 8;
+  for (int base = 0; base < nO && cnt < nI; base += 64 * kSearch) {
+    bool in[kSearch];
+    long long t[kSearch];
+#pragma unroll
+    for (int r = 0; r < kSearch; ++r) {
+      const int o = base + 64 * r + lane;
+      in[r] = o < nO;
+      t[r] = 0;
+      long long mul = 1;
       for (int d = 0; d < D; ++d) {
-        int x = cc[d] + offs[(long long)o * D + d];
+        int x = cc[d] + offs[(long long)(o0 + min(o, nO - 1)) * D + d];
         // include/simulation.hpp:394: `|| circularSim` takes the wrapped cell
         if (circSim) x = ((x % sd[d]) + sd[d]) % sd[d];
-        inside &= (x >= 0 && x < sd[d]);
-        t += (long long)x * mul;
+        in[r] &= (x >= 0 && x < sd[d]);
+        t[r] += (long long)x * mul;
         mul *= sd[d];
       }
-      if (inside) {
-        pj = postS[t];
-        hit = pj <= (int)i;
+    }
+    int pj[kSearch];
+#pragma unroll
+    for (int r = 0; r < kSearch; ++r) pj[r] = postS[in[r] ? t[r] : 0];
+#pragma unroll
+    for (int r = 0; r < kSearch; ++r) {
+      const bool hit = in[r] && pj[r] <= (int)i;
+      const unsigned long long m = __ballot(hit);
+      const int before = __popcll(m & ((1ull << lane) - 1ull));
+      if (hit && cnt + before < nI) {
+        out[cnt + before] = o0 + base + 64 * r + lane;
+        outP[cnt + before] = pj[r];
       }
+      cnt += __popcll(m);
     }
-    const unsigned long long m = __ballot(hit);
-    const int before = __popcll(m & ((1ull << lane) - 1ull));
-    if (hit && cnt + before < nI) {
-      out[cnt + before] = o;
-      outP[cnt + before] = pj;
-    }
-    cnt += __popcll(m);
   }
   if (lane == 0) nbCnt[i] = min(cnt, nI);
 }
