@@ -1318,6 +1318,10 @@ static int flow_slices(const FlowPlan& F, long long S, int terms) {
   return (int)std::max<long long>(1, std::min<long long>(48, pairs / per));
 }
 
+// Nodes after which FlowPlan::waveUs is compared with the time they took: the
+// first and slowest ones, whose neighbours are far.
+constexpr int kFlowJudge = 65536;
+
 int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, bool* gaveUp) {
   hipStream_t st = t->stream;
   *gaveUp = false;
@@ -1436,7 +1440,8 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   double ms = 0.0;
   const auto begun = std::chrono::steady_clock::now();
   auto told = begun;
-  for (size_t b = 0; b < nPath && e == hipSuccess; b += seg) {
+  bool slow = false, judged = !(F.waveUs > 0.0);
+  for (size_t b = 0; b < nPath && e == hipSuccess && !slow; b += seg) {
     P.node0 = (int)b;
     P.nNodes = (int)std::min(seg, nPath - b);
     if (b) e = hipMemsetAsync(P.ctl, 0, sizeof(int), st);  // the ticket
@@ -1462,11 +1467,17 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
       float one = 0.f;
       if (hipEventSynchronize(ev[1]) == hipSuccess && hipEventElapsedTime(&one, ev[0], ev[1]) == hipSuccess) ms += one;
     }
+    const size_t done = b + (size_t)P.nNodes;
+    if (!judged && done >= (size_t)kFlowJudge && hipStreamSynchronize(st) == hipSuccess) {
+      judged = true;
+      slow = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - begun).count() >
+             F.waveUs * (double)done;
+    }
     if (R.progressSec > 0 && hipStreamSynchronize(st) == hipSuccess) {
       const auto now = std::chrono::steady_clock::now();
       if (std::chrono::duration<double>(now - told).count() >= R.progressSec) {
         told = now;
-        std::fprintf(stderr, "[qsmi] path loop: %zu of %zu nodes done, %.0f s\n", b + (size_t)P.nNodes, nPath,
+        std::fprintf(stderr, "[qsmi] path loop: %zu of %zu nodes done, %.0f s\n", done, nPath,
                      std::chrono::duration<double>(now - begun).count());
         std::fflush(stderr);
       }
@@ -1483,7 +1494,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   if (e == hipSuccess) e = hipMemcpy(ctl, P.ctl, sizeof(ctl), hipMemcpyDeviceToHost);
   if (e == hipSuccess) e = hipMemcpy(sv, P.stats, sizeof(sv), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return fail(QSMI_ERR_HIP, std::string("path loop: ") + hipGetErrorString(e));
-  *gaveUp = ctl[1] != 0;
+  *gaveUp = ctl[1] != 0 || slow;
   *kernelMs = ms;
   for (int q = 0; q < 4; ++q) stats[q] = (long long)sv[q];
   return QSMI_OK;

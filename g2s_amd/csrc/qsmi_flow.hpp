@@ -19,11 +19,13 @@ struct FlowPlan {
   float rare[kFlowMaxCat] = {};                // per class: 1 - its share of the TI
   int inFlight = 1 << 20;  // path nodes simulated at the same time, at most
   int segment = 65536;     // path nodes per launch
+  double waveUs = 0.0;     // microseconds a node above which the wave loop is the faster one (0: never)
 };
 
 // Simulates the path (R's neighbour lists, grid and tables on the device).
 // stats: exact-selection nodes, rescored positions, 0, list flushes.
-// gaveUp: a wait hit its bound; the grid is not usable then.
+// gaveUp: a wait hit its bound, or the first nodes took longer than waveUs
+// each; the grid is not usable then.
 int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, bool* gaveUp);
 
 }  // namespace qsmi

@@ -987,11 +987,24 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
         flow.inFlight = rq->waveSize;
         flow.segment = (int)std::min<long long>(flow.segment, 64ll * rq->waveSize);
       }
+      // The wave loop's transforms cost the same for every image, the direct
+      // scan less the sooner its bound rules a position out. On the 1024 x
+      // 1024 grid, the one where the transforms come close, 80 neighbours and
+      // full waves take 3.25 us a node (250 neighbours 5.1) and the direct
+      // scan of a 1000 x 1000 image 2.9 (correlation length 20), 3.5 (8), 4.3
+      // (3) and 5.0 (white noise); its first 65536 nodes take 3.1, 4.3, 5.9
+      // and 6.2. Starting over pays above 4.6, where the path is long enough
+      // for that and its levels wide enough to fill waves: noise then takes
+      // 3.24 s + 0.4 s instead of 5.0. On every other grid the direct scan
+      // stays ahead in noise too (500 x 500: 1.8 us a node against 3.3).
+      if (D == 2 && ti->w1k && nVar == 1 && !flow.count && nPath >= 4 * 65536 && flow.inFlight >= 256 &&
+          S > 600 * 1000)
+        flow.waveUs = 4.6 + 0.011 * std::max(0, nMax - 80);
       bool gaveUp = false;
       rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &gaveUp);
       scanned = (long long)nPath;
       waves = (int)R.waveLevel.size();
-      if (!rc && gaveUp) {  // a device wait hit its bound: the wave loop, from the start
+      if (!rc && gaveUp) {  // the wave loop, from the start
         for (void* p : allocs) (void)hipFree(p);
         qsmi_ti_destroy(ti);
         return qs_run(rq, rs, false);

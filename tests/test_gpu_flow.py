@@ -114,3 +114,20 @@ def test_flow_slices_and_segments():
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     flow, waves = _both(ti, dims, di, sdims, [0], 24, 1.5, 4, wave_size=64)
     assert flow["exact_nodes"] == waves["exact_nodes"]
+
+
+def test_flow_hands_over_to_waves():
+    """White noise on the 1024 grid: the first nodes take longer than the wave
+    loop's, which starts over (or the data-flow loop goes on: same bytes)."""
+    rng = np.random.default_rng(8)
+    dims, sdims = (1000, 1000), (530, 500)
+    ti = rng.standard_normal(dims[0] * dims[1]).astype(np.float32)
+    di = np.full(sdims[0] * sdims[1], np.nan, np.float32)
+    out = []
+    try:
+        for flow in (1, 0):
+            g2s_amd.set_default_tuning("loop.flow", flow)
+            out.append(g2s_amd.qs(ti, dims, di, sdims, [0], 80, 1.5, 6))
+    finally:
+        g2s_amd.set_default_tuning("loop.flow", 1)
+    assert out[0][0].tobytes() == out[1][0].tobytes() and out[0][1].tobytes() == out[1][1].tobytes()
