@@ -128,6 +128,14 @@ struct qsmi_device {
   // map holds a value set from outside (then the FP32 selection is kept)
   NodeInfo lastNode{};
   bool mapEdited = false;
+  // the direct sum (qsmi_node.hip): the FP64 map, whether it is the current
+  // map's, the scale it was made with, chunk results, and the K best in pinned
+  // host memory
+  double* dMapD = nullptr;
+  bool mapExact = false;
+  int mapScaled = 0;
+  qsmi::Cand64* dPart = nullptr;
+  uint32_t* hBest = nullptr;
   BandBufs band;
   // second stream of the resident loop (consecutive waves of one dependency
   // level alternate between stream and side.stream), with its own wave

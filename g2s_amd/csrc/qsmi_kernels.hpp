@@ -68,6 +68,15 @@ struct NodeInfo {
                       // value is rescored in FP64 before the device rule picks the K best)
 };
 
+// One node of the per-node API as kernel arguments: nb * D offsets, then the
+// bits of nb * V combined values (both within the 4 KiB that a launch passes).
+constexpr int kNodeWords = 768;
+constexpr int kNodeChunks = 512;
+struct NodeArgs {
+  NodeInfo ni;
+  int w[kNodeWords];
+};
+
 // Several TIs: the first cell of each TI in their concatenation, then the total.
 struct TiCum {
   unsigned c[9];

@@ -1,0 +1,105 @@
+"""The direct sum of the per-node API against plain FP64 on the host and
+against the wave scan, the general path of the same nodes: the map is the FP64
+value rounded to FP32 (half a unit in the last place), and the K best are the
+same positions and values. Sizes around a wavefront's and a block's run, both
+widths of the kernel (below and above 2^19 positions), 1-3 dimensions, one,
+two and more sub-images, crowded ties, exclusions, and the two forms of the
+selection on one map."""
+import numpy as np
+import pytest
+
+import g2s_amd
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # dims, variable types, neighbours, K, values
+    ((63,), [0], 3, 1, "cont"),
+    ((64, 5), [0], 1, 2, "cont"),
+    ((257, 4), [0], 9, 3, "cont"),
+    ((33, 31), [0], 8, 16, "steps"),
+    ((40, 30), [0], 17, 2, "flat"),
+    ((21, 13, 9), [0], 30, 5, "cont"),
+    ((50, 41), [0, 0], 12, 2, "cont"),
+    ((45, 37), [0, 1], 20, 4, "cont"),
+    ((725, 724), [0], 25, 2, "cont"),
+    ((1000, 1000), [0], 80, 2, "cont"),
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_node_direct(case):
+    dims, types, n, K, kind = CASES[case]
+    print(f"direct node: case {case} {CASES[case]}", flush=True)
+    rng = np.random.default_rng(40 + case)
+    S = int(np.prod(dims))
+    ti = rng.standard_normal((S, len(types)))
+    if kind == "steps":
+        ti = np.round(ti)
+    if kind == "flat":
+        ti[:] = 0.5
+    for v, t in enumerate(types):
+        if t:
+            ti[:, v] = rng.integers(0, 3, S)
+    ti = ti.astype(np.float32)
+    cats = [g2s_amd.categories(ti, len(types), v) for v, t in enumerate(types) if t]
+    ncat = [len(c) for c in cats]
+    sub = g2s_amd.ti_subimages(ti, dims, types, ncat, [x for c in cats for x in c])
+    alpha = g2s_amd.coef_matrix(types, ncat)[0]
+    image = g2s_amd.TrainingImage(sub, dims)
+    dev = g2s_amd.AcceleratorDevice(image, alpha)
+    nsub = sub.reshape(-1, S).shape[0]
+    D = len(dims)
+    shape = tuple(reversed(dims))
+    for trial in range(2):
+        off = np.stack([rng.integers(-min(6, d // 4), min(6, d // 4) + 1, n) for d in dims], 1).astype(np.int32)
+        vals = rng.standard_normal((n, nsub)).astype(np.float32)
+        d0 = float(np.float32(-3.25))
+        seed = float(np.float32(rng.random()))
+        assert dev.candidate_for_pattern(off, vals, d0)
+        got = dev.error_map().reshape(shape)
+        # FP64: v_ja = sum_B alpha(A, B) u_jB in FP32 as the library combines
+        v = np.zeros((n, nsub), np.float32)
+        for b in range(nsub):
+            v = v + alpha[:, b][None, :].astype(np.float32) * vals[:, b:b + 1]
+        lo = [max(0, -int(off[:, d].min())) for d in range(D)]
+        hi = [dims[d] - 1 - max(0, int(off[:, d].max())) for d in range(D)]
+        want = np.full(shape, -np.inf)
+        box = tuple(slice(lo[d], hi[d] + 1) for d in reversed(range(D)))
+        acc = np.full(want[box].shape, d0)
+        img = sub.reshape((nsub,) + shape).astype(np.float64)
+        size = np.abs(acc)
+        for j in range(n):
+            at = tuple(slice(lo[d] + off[j, d], hi[d] + 1 + off[j, d]) for d in reversed(range(D)))
+            for a in range(nsub):
+                acc = acc + float(v[j, a]) * img[a][at]
+                size = size + np.abs(float(v[j, a]) * img[a][at])
+        want[box] = acc
+        assert np.array_equal(np.isfinite(got), np.isfinite(want))
+        fin = np.isfinite(want)
+        bound = np.zeros(shape)
+        # one rounding to FP32, and FP32 combinations of nsub terms a value
+        bound[box] = np.abs(acc) * 2.0 ** -24 + size * (nsub * 2.0 ** -23 if nsub > 2 else 2.0 ** -40)
+        assert np.all(np.abs(got - want)[fin] <= bound[fin] + 1e-30)
+        e, i = dev.search_k_biggest(K, seed)
+        e2, i2 = dev.search_k_biggest_noalloc(K, seed)
+        assert np.array_equal(i, i2) and np.array_equal(e, e2)
+        we, wp = dev.scan_wave([(off, vals, d0, seed)], K)[:2]
+        pos = [dev.cvt_index_to_position(int(q)) if q != 0xFFFFFFFF else 0xFFFFFFFF for q in i]
+        assert list(np.asarray(wp).reshape(-1)[:K]) == pos
+        assert np.array_equal(np.asarray(we).reshape(-1)[:K], e)
+        # an exclusion, then a finite value: the best position goes, then wins
+        if i[0] != 0xFFFFFFFF:
+            dev.set_value_in_error_array(int(i[0]), -np.inf)
+            e3, i3 = dev.search_k_biggest(K, seed)
+            assert i[0] not in i3
+            dev.set_value_in_error_array(int(i[0]), 1e9)
+            assert dev.search_k_biggest(K, seed)[1][0] == i[0]
+    # no valid position
+    off = np.zeros((2, D), np.int32)
+    off[0, 0], off[1, 0] = dims[0] // 2 + 1, -(dims[0] // 2 + 1)
+    assert dev.candidate_for_pattern(off, np.ones((2, nsub), np.float32), 0.0)
+    assert not np.isfinite(dev.error_map()).any()
+    assert np.all(dev.search_k_biggest(K, 0.5)[1] == 0xFFFFFFFF)
+    dev.close()
+    image.close()
