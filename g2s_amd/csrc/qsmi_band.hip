@@ -28,7 +28,7 @@
 //      of 64 positions spread over one grid, so a crowded node's list is
 //      scored by as many wavefronts as it has tiles. A node whose band
 //      overflows the list capacity (full fallback) is rescored over its whole
-//      valid box instead, in kFullTiles tiles that keep their K best.
+//      valid box instead, in tiles that keep their K best.
 //   4. k_band_final: per node, the K best by the device rule on the FP64
 //      values, then the rank draw and the simulation write.
 // Nodes with eps == 0 (categorical-only TIs with a tie quantum, TIs with
@@ -59,7 +59,13 @@ void launch_rows_collect(const ScanGeom& g, const FftPlan& plan0, int lognv, con
 namespace {
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
-constexpr int kFullTiles = 128;  // rescoring tiles of a full-fallback node (slices of its valid box)
+// Rescoring tiles of a full-fallback node (slices of its valid box), one
+// wavefront each: a node's box is a serial chain of box / tiles / 64 rounds,
+// so the tail of a wave with one such node is set by their number. 128 -> 1024
+// tiles: 234 -> 67 us a launch of the calibration (1000 x 1000).
+// The per-GPU scratch array of the allocation-free search holds 128.
+constexpr int kFullTiles = 1024;
+constexpr int kFullTilesScratch = 128;
 constexpr int kSegNodes = 2048;  // nodes per rescoring launch (their tile prefix sums are held in LDS)
 
 // Device view of the band buffers.
@@ -70,7 +76,8 @@ struct BandDev {
   int2* queue;     // (node, rows block) items of the second pass
   int* qcnt;       // [0] queue items (zero between calls)
   double* val;     // [node][kBandCap] FP64 values of the listed positions
-  Cand64* part;    // [node][kFullTiles][K] full-fallback tile results
+  Cand64* part;    // [node][tiles][K] full-fallback tile results
+  int tiles;       // tiles of a full-fallback node
   unsigned long long* stats;  // exact nodes, listed positions, second-pass blocks, full-fallback nodes
 };
 
@@ -83,6 +90,7 @@ BandDev dev_view(const BandBufs& b) {
   d.qcnt = b.qcnt;
   d.val = b.val;
   d.part = b.part;
+  d.tiles = b.tiles;
   d.stats = b.stats;
   return d;
 }
@@ -297,8 +305,8 @@ __global__ void __launch_bounds__(256) k_merge_band(const NodeInfo* __restrict__
   }
 }
 
-__device__ __forceinline__ int band_tiles(int cnt) {
-  return cnt < 0 ? 0 : cnt > kBandCap ? kFullTiles : (cnt + 63) >> 6;
+__device__ __forceinline__ int band_tiles(int cnt, int tiles) {
+  return cnt < 0 ? 0 : cnt > kBandCap ? tiles : (cnt + 63) >> 6;
 }
 
 // Step 3. Nodes [node0, node0 + nSeg) (nSeg <= kSegNodes), one wavefront
@@ -322,7 +330,7 @@ __global__ void __launch_bounds__(64) k_band_rescore(ScanGeom g, const NodeInfo*
   const int per = (nLive + 63) >> 6;
   const int r0 = min(nLive, tid * per), r1 = min(nLive, r0 + per);
   int run = 0;
-  for (int i = r0; i < r1; ++i) run += band_tiles(bb.cnt[node0 + i]);
+  for (int i = r0; i < r1; ++i) run += band_tiles(bb.cnt[node0 + i], bb.tiles);
   int incl = run;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
@@ -332,7 +340,7 @@ __global__ void __launch_bounds__(64) k_band_rescore(ScanGeom g, const NodeInfo*
   int acc = incl - run;
   for (int i = r0; i < r1; ++i) {
     pre[i] = acc;
-    acc += band_tiles(bb.cnt[node0 + i]);
+    acc += band_tiles(bb.cnt[node0 + i], bb.tiles);
   }
   if (tid == 63) pre[nLive] = incl;
   __syncthreads();
@@ -366,7 +374,7 @@ __global__ void __launch_bounds__(64) k_band_rescore(ScanGeom g, const NodeInfo*
     } else {  // the list overflowed: slice lt of the whole valid box
       const long long n0 = ni.hi[0] - ni.lo[0] + 1, n1 = ni.hi[1] - ni.lo[1] + 1, n2 = ni.hi[2] - ni.lo[2] + 1;
       const long long box = (n0 > 0 && n1 > 0 && n2 > 0) ? n0 * n1 * n2 : 0;
-      const long long len = (box + kFullTiles - 1) / kFullTiles;
+      const long long len = (box + bb.tiles - 1) / bb.tiles;
       const long long beg = (long long)lt * len, end = min(box, beg + len);
       TopK64<KT> tk;
       tk.init();
@@ -382,7 +390,7 @@ __global__ void __launch_bounds__(64) k_band_rescore(ScanGeom g, const NodeInfo*
         c.pos = p;
         tk.push(c);
       }
-      block_topk64<KT>(tk, K, bb.part + ((long long)node * kFullTiles + lt) * K, red);
+      block_topk64<KT>(tk, K, bb.part + ((long long)node * bb.tiles + lt) * K, red);
     }
   }
 }
@@ -422,8 +430,8 @@ __global__ void __launch_bounds__(256) k_band_final(const NodeInfo* __restrict__
     }
     if (tid == 0) atomicAdd(&bb.stats[1], (unsigned long long)cnt);
   } else {
-    const Cand64* pp = bb.part + (long long)node * kFullTiles * K;
-    for (int i = tid; i < kFullTiles * K; i += blockDim.x) tk.push(pp[i]);
+    const Cand64* pp = bb.part + (long long)node * bb.tiles * K;
+    for (int i = tid; i < bb.tiles * K; i += blockDim.x) tk.push(pp[i]);
     if (tid == 0) atomicAdd(&bb.stats[3], 1ull);
   }
   block_topk64<KT>(tk, K, best, red);
@@ -531,6 +539,7 @@ int band_grow(BandBufs* b, int nNodes, int blocksPerNode, int K) {
     band_free(b);
     return fail(QSMI_ERR_NOMEM, "exact selection buffers: out of device memory");
   }
+  b->tiles = kFullTiles;
   b->capNodes = nn;
   b->capQueue = qq;
   b->K = kk;
@@ -543,7 +552,7 @@ int band_grow(BandBufs* b, int nNodes, int blocksPerNode, int K) {
 size_t band_scratch_bytes(int K) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   return al(kBandCap * sizeof(uint32_t)) + 2 * al(sizeof(int)) + al(sizeof(float)) + al(sizeof(int2)) +
-         al(kBandCap * sizeof(double)) + al((size_t)kFullTiles * K * sizeof(Cand64)) +
+         al(kBandCap * sizeof(double)) + al((size_t)kFullTilesScratch * K * sizeof(Cand64)) +
          al(4 * sizeof(unsigned long long));
 }
 
@@ -563,8 +572,9 @@ void band_view(BandBufs* b, void* base, int K) {
   b->val = reinterpret_cast<double*>(p);
   p += al(kBandCap * sizeof(double));
   b->part = reinterpret_cast<Cand64*>(p);
-  p += al((size_t)kFullTiles * K * sizeof(Cand64));
+  p += al((size_t)kFullTilesScratch * K * sizeof(Cand64));
   b->stats = reinterpret_cast<unsigned long long*>(p);
+  b->tiles = kFullTilesScratch;
   b->capNodes = 1;
   b->capQueue = 1;
   b->K = K;
@@ -595,7 +605,7 @@ void launch_rescore(const ScanGeom& g, const NodeInfo* info, const int* nbOff, c
     const int nSeg = std::min(kSegNodes, nNodes - n0);
     // about two tiles per node (most lists hold under 64 positions); blocks
     // beyond the tile total return after the prefix
-    const int grid = std::min(8192, 2 * nSeg + 512);
+    const int grid = std::min(8192, 2 * nSeg + 1024);
     hipLaunchKernelGGL(k_band_rescore<KT>, dim3((unsigned)grid), dim3(64), lds, st, g, info, nbOff, nbVal, t->dSub,
                        t->S, nscale, K, n0, nSeg, bd, count);
   }

@@ -66,7 +66,8 @@ struct BandBufs {
   int2* queue = nullptr;         // second-pass items (node, rows block)
   int* qcnt = nullptr;           // [2]: queue items (zero between calls), unused
   double* val = nullptr;         // [node][kBandCap] FP64 values of the listed positions
-  qsmi::Cand64* part = nullptr;  // [node][kFullTiles][K] full-fallback tile results
+  qsmi::Cand64* part = nullptr;  // [node][tiles][K] full-fallback tile results
+  int tiles = 0;
   unsigned long long* stats = nullptr;  // exact nodes, listed positions, second-pass blocks, full-fallback nodes
 };
 
