@@ -21,14 +21,15 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-PROFILE = "profiles/k_pencil1024__qs_2d_continuous_1000.md"
+PROFILES = {"k_pencil1024": "profiles/k_pencil1024__qs_2d_continuous_1000.md",
+            "k_flow_direct": "profiles/k_flow_direct__qs_2d_continuous_1000.md"}
 
 
 def measured_bytes_per_node(kernel):
     """HBM bytes per node of `kernel` (calibrated FETCH_SIZE + WRITE_SIZE)
     from the committed rocprofv3 counter summary, or None."""
     try:
-        with open(os.path.join(ROOT, PROFILE)) as fh:
+        with open(os.path.join(ROOT, PROFILES[kernel])) as fh:
             for line in fh:
                 if line.startswith(f"hbm_bytes_per_node {kernel}:"):
                     f, w = line.split(":", 1)[1].split()
@@ -53,7 +54,7 @@ def parse():
     ap.add_argument("--wave", type=int, default=256,
                     help="max path nodes per wave: the workload batches 256 path nodes per launch")
     ap.add_argument("--stage-every", type=int, default=32,
-                    help="HIP events around the stages of every k-th wave of the timed steps (1: every wave; "
+                    help="wave loop: HIP events around the stages of every k-th wave of the timed steps (1: every wave; "
                          "events cost ~1.5%% of the loop when recorded for every wave)")
     ap.add_argument("--graph-steps", type=int, default=1,
                     help="also time the step with each wave replayed as a captured HIP graph (0: skip)")
@@ -423,31 +424,43 @@ def main():
     nodes = stats[-1]["nodes"]
     ms = float(np.mean(times))
     value = nodes / (ms / 1e3)
-    # roofline of the dominant kernel (the fused spectrum stage): algorithmic
-    # bytes per node A = V*S*8 + 2*N*4 (V=2 spectra of S=501*1000 complex64,
-    # N=10^6 map floats written and read) over its event-timed duration
+    # roofline of the dominant kernel: algorithmic bytes per node
+    # A = V*S*8 + 2*N*4 (V=2 spectra of S=501*1000 complex64, N=10^6 map
+    # floats written and read: a scan by transforms) over its event-timed
+    # duration. The data-flow loop (no gather stage of its own) is one kernel,
+    # launched once for 64 waves of nodes; the wave loop's dominant kernel is
+    # the spectrum stage, launched once a wave.
     V, S, N = 2, (dims[0] // 2 + 1) * dims[1], dims[0] * dims[1]
     a_node = V * S * 8 + 2 * N * 4
     st = stats[-1]
-    pencil_ms = st.get("spectrum_ms", 0.0)
+    kernel_ms = st.get("spectrum_ms", 0.0)
     roof = None
-    if pencil_ms > 0:
-        achieved = a_node * st["scanned_nodes"] / (pencil_ms / 1e3) / 1e9
-        nodes_per_launch = st["scanned_nodes"] / max(1, st["waves"])
-        per_node = measured_bytes_per_node("k_pencil1024") if dims == (1000, 1000) else None
+    if kernel_ms > 0:
+        flow = st["gather_ms"] == 0.0
+        kernel = "k_flow_direct" if flow else "k_pencil1024"
+        launches = max(1, -(-st["scanned_nodes"] // min(65536, 64 * args.wave)) if flow else st["waves"])
+        achieved = a_node * st["scanned_nodes"] / (kernel_ms / 1e3) / 1e9
+        nodes_per_launch = st["scanned_nodes"] / launches
+        per_node = measured_bytes_per_node(kernel) if dims == (1000, 1000) else None
+        if flow:
+            timing = "HIP events around every launch of the timed step"
+            note = ("the algorithmic bytes are those of a scan by transforms; the kernel sums the map's terms "
+                    "directly and drops positions by a running bound, from the TI in the caches: it is bound by "
+                    "VALU and scalar issue and L1, and traffic is its measured HBM bytes per launch")
+        else:
+            timing = (f"HIP events on the stream of every {args.stage_every}-th wave of the timed "
+                      "step (k_taps work included with the gather)")
+            note = ("the algorithmic bytes count a 4-byte map per TI cell written and read once; the "
+                    "pencil and rows kernels never materialise that map (column transforms pass between "
+                    "them), so achieved may exceed the HBM peak: the pencil is bound by VALU issue, and "
+                    "traffic is its measured HBM bytes per launch. Consecutive waves of one dependency level "
+                    "run on two streams, so a launch's duration includes time shared with the other "
+                    "stream's kernels")
         roof = dict(bound="hbm", achieved=achieved, peak=HBM_PEAK_GBS, unit="GB/s", frac=achieved / HBM_PEAK_GBS,
                     traffic=(per_node * nodes_per_launch if per_node else None),
-                    kernel="k_pencil1024", avg_launch_us=pencil_ms * 1e3 / max(1, st["waves"]),
+                    kernel=kernel, avg_launch_us=kernel_ms * 1e3 / launches,
                     nodes_per_launch=nodes_per_launch, algorithmic_bytes_per_node=a_node,
-                    traffic_source=(PROFILE if per_node else None),
-                    launch_timing=(f"HIP events on the stream of every {args.stage_every}-th wave of the timed "
-                                   "step (k_taps work included with the gather)"),
-                    note=("the algorithmic bytes count a 4-byte map per TI cell written and read once; the "
-                          "pencil and rows kernels never materialise that map (column transforms pass between "
-                          "them), so achieved may exceed the HBM peak: the pencil is bound by VALU issue, and "
-                          "traffic is its measured HBM bytes per launch. Consecutive waves of one dependency level "
-                          "run on two streams, so a launch's duration includes time shared with the other "
-                          "stream's kernels"))
+                    traffic_source=(PROFILES[kernel] if per_node else None), launch_timing=timing, note=note)
     alt = None
     if args.alt_wave > 0 and args.alt_wave != args.wave:
         _, _, sa = g2s_amd.qs(ti, dims, di, sdims, cfg["types"], n, k, seed=cfg["seed"], wave_size=args.alt_wave,

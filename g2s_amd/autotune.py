@@ -10,8 +10,12 @@ tuning keys (``qsmi_set_default_tuning``) and keeps the fastest:
   the transforms per FFT block (``fft.lognv_max``) and the path nodes per
   pencil block (``pencil.npb``), one key after the other (coordinate
   descent from the defaults);
-* on the 1024 x 1024 grid: launched kernels against one captured HIP graph
-  per wave step (``loop.graph``).
+* on the 1024 x 1024 grid: the path loop as it is chosen by itself (the
+  data-flow loop where the request allows it, else launched waves) against
+  one captured HIP graph per wave step (``loop.graph``).
+
+The first two concern scans by transforms, which the data-flow loop does not
+run: their probes take the wave loop (``loop.flow`` 0).
 
 Choices are cached in a JSON file keyed by the geometry; a later call with
 the same cache reads the choice instead of measuring again. The choice is
@@ -21,13 +25,14 @@ with a continuous variable the exact selection makes the realisation
 independent of them; categorical-only TIs keep the FP32 selection, whose ties
 within the quantum may then resolve differently.
 """
+import contextlib
 import json
 import os
 import tempfile
 
 import numpy as np
 
-from . import qs, set_default_tuning
+from . import TrainingImage, qs, set_default_tuning
 
 DEFAULTS = {"scan.grid1024_min": 320, "fft.radix_max": 13, "fft.lognv_max": 6, "pencil.npb": 1, "loop.graph": 0}
 OWN_GRID_CANDIDATES = (("fft.radix_max", (13, 8, 5)), ("fft.lognv_max", (6, 4, 3)), ("pencil.npb", (1, 2, 4)))
@@ -77,11 +82,22 @@ def _probe_run(ti, ti_dims, var_types, n, k, sim_dims, seed):
     return st["path_loop_ms"]
 
 
-def _time(settings, ti, ti_dims, var_types, n, k, sim_dims, repeats, seed):
+def _default_flow():
+    """The default of loop.flow: what a TI created now starts with."""
+    with contextlib.closing(TrainingImage(np.zeros((1, 4), np.float32), (2, 2))) as image:
+        return image.get_tuning("loop.flow")
+
+
+def _time(settings, flow, ti, ti_dims, var_types, n, k, sim_dims, repeats, seed):
     apply(settings)
-    _probe_run(ti, ti_dims, var_types, n, k, sim_dims, seed)  # kernels loaded, buffers sized
-    return float(np.median([_probe_run(ti, ti_dims, var_types, n, k, sim_dims, seed + 1 + r)
-                            for r in range(repeats)]))
+    before = _default_flow()
+    try:
+        set_default_tuning("loop.flow", min(flow, before))
+        _probe_run(ti, ti_dims, var_types, n, k, sim_dims, seed)  # kernels loaded, buffers sized
+        return float(np.median([_probe_run(ti, ti_dims, var_types, n, k, sim_dims, seed + 1 + r)
+                                for r in range(repeats)]))
+    finally:
+        set_default_tuning("loop.flow", before)
 
 
 def autotune(ti, ti_dims, var_types, n, k, cache=None, sim_dims=None, repeats=3, seed=7):
@@ -101,8 +117,8 @@ def autotune(ti, ti_dims, var_types, n, k, cache=None, sim_dims=None, repeats=3,
     best = dict(DEFAULTS)
     measured = {}
 
-    def trial(label, cand):
-        t = _time(cand, ti, ti_dims, var_types, n, k, sim_dims, repeats, seed)
+    def trial(label, cand, flow=0):
+        t = _time(cand, flow, ti, ti_dims, var_types, n, k, sim_dims, repeats, seed)
         measured[label] = t
         return t
 
@@ -113,7 +129,7 @@ def autotune(ti, ti_dims, var_types, n, k, cache=None, sim_dims=None, repeats=3,
         own_grid = town <= t1024
         best["scan.grid1024_min"] = 1025 if own_grid else 2
     if not own_grid:
-        times = {v: trial(f"loop.graph={v}", dict(best, **{"loop.graph": v})) for v in (0, 1)}
+        times = {v: trial(f"loop.graph={v}", dict(best, **{"loop.graph": v}), flow=1) for v in (0, 1)}
         best["loop.graph"] = min(times, key=times.get)
     if own_grid:
         for tkey, values in OWN_GRID_CANDIDATES:

@@ -102,8 +102,13 @@ int qsmi_ti_destroy(qsmi_ti* ti);
  *                 wave's kernels as one captured HIP graph per stream (plain
  *                 1024-grid scans with the two-stream loop; the sampled
  *                 stage timing is not recorded then): 0..1, default 0
+ *   "loop.flow"   1: the path loop runs as one persistent kernel that
+ *                 simulates every node as soon as its neighbours hold values,
+ *                 without transforms, where the request allows it (one TI,
+ *                 not circular, no NaN, no learned proposal, record or -nV;
+ *                 loop.graph 0): 0..1, default 1; 0: waves of transforms
  * Results do not depend on them up to the FP32 map error the exact selection
- * absorbs (pencil.npb, loop.graph: every choice gives the same bytes).
+ * absorbs (pencil.npb, loop.graph, loop.flow: every choice gives the same bytes).
  * QSMI_ERR_ARG for an unknown key or a value out of range. */
 int qsmi_ti_set_tuning(qsmi_ti* ti, const char* key, int value);
 int qsmi_ti_get_tuning(const qsmi_ti* ti, const char* key, int* value);
@@ -153,7 +158,9 @@ int qsmi_candidate_for_pattern(qsmi_device* dev, int nNeighbors, const int* offs
  * (eps = 4e-5 * sum_a rms(Y_a) * sum_j |v_ja|, the bound of the FP32 map
  * error: rms over the FFT grid of TI sub-image a, v_ja the neighbours'
  * alpha-combined values) is rescored in FP64 and the extendK best of those
- * values are returned (as floats). After a finite value was set with
+ * values are returned (as floats); where the map was summed directly in FP64
+ * (not circular, no cross layer, at most 2^29 terms) its values are ranked as
+ * they are, the same result. After a finite value was set with
  * qsmi_set_value_in_error_array(_with_radius) the FP32 map is used as is. */
 int qsmi_search_k_biggest(qsmi_device* dev, float* errors, unsigned* encodedPosition, unsigned extendK, float seed);
 
