@@ -1007,7 +1007,15 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
       if (!rc && gaveUp) {  // the wave loop, from the start
         for (void* p : allocs) (void)hipFree(p);
         qsmi_ti_destroy(ti);
-        return qs_run(rq, rs, false);
+        const double setup = std::chrono::duration<double, std::milli>(t1 - t0).count();
+        const double lost = std::chrono::duration<double, std::milli>(clk::now() - t1).count();
+        rc = qs_run(rq, rs, false);
+        if (!rc) {  // what the first attempt took counts
+          rs->setupMs += setup;
+          rs->pathLoopMs += lost;
+          rs->phaseMs[3] += lost;
+        }
+        return rc;
       }
     } else {
       rc = qsmi::run_resident_waves(dev, R, stageMs, &scanned, &waves, bandStats);
