@@ -72,7 +72,6 @@ constexpr int kTileX = 16, kTileY = 4, kPair = 2, kRun = 16;
 constexpr int kStep = 8;        // terms between two looks at the bound
 constexpr int kWaveList = 256;  // kept positions of a wavefront before they are scored
 constexpr int kSources = 32;    // neighbours whose source positions seed the bound
-constexpr int kPolls = 1 << 22;  // x s_sleep(2) (128 cycles): ~0.3 s and more, far above any real wait
 
 struct FlowParams {
   int D, nVar, nExp, n, K, G, circSim;
@@ -102,7 +101,8 @@ struct FlowParams {
   const float* di;    // the grid as given
   uint32_t* work;     // the grid under simulation
   uint32_t* index;
-  int* ctl;           // [0] ticket, [1] error
+  int* ctl;           // [0] ticket, [1] a wait was given up
+  int polls;          // polls after which a wait is given up
   unsigned long long* slots;
   unsigned long long* stats;
   int node0, nNodes;
@@ -131,10 +131,10 @@ __device__ __forceinline__ void st_agent64(unsigned long long* p, unsigned long 
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Bounded wait step: false when the wait is given up (then *err is set and
-// every other wait of the kernel ends as well).
-__device__ __forceinline__ bool poll_again(int& polls, int* err) {
-  if (++polls >= kPolls) {
+// Bounded wait step: false when the wait is given up (then *err is set, every
+// other wait of the kernel ends as well and no block takes another ticket).
+__device__ __forceinline__ bool poll_again(int& polls, int bound, int* err) {
+  if (++polls >= bound) {
     st_agent((uint32_t*)err, 1u);
     return false;
   }
@@ -143,19 +143,19 @@ __device__ __forceinline__ bool poll_again(int& polls, int* err) {
   return true;
 }
 
-__device__ __forceinline__ uint32_t wait_word(const uint32_t* p, int* err) {
+__device__ __forceinline__ uint32_t wait_word(const uint32_t* p, int bound, int* err) {
   uint32_t b = ld_agent(p);
   for (int polls = 0; b == kPending;) {
-    if (!poll_again(polls, err)) return kEmpty;
+    if (!poll_again(polls, bound, err)) return kEmpty;
     b = ld_agent(p);
   }
   return b;
 }
 
-__device__ __forceinline__ unsigned long long wait_word64(const unsigned long long* p, int* err) {
+__device__ __forceinline__ unsigned long long wait_word64(const unsigned long long* p, int bound, int* err) {
   unsigned long long b = ld_agent64(p);
   for (int polls = 0; b == kOpen;) {
-    if (!poll_again(polls, err)) return kOpen;
+    if (!poll_again(polls, bound, err)) return kOpen;
     b = ld_agent64(p);
   }
   return b;
@@ -165,6 +165,13 @@ __device__ __forceinline__ uint32_t seed_bits_of(float seed) {
   if (!isfinite(seed) || seed <= 0.f) return 0u;
   if (seed >= 1.f) return 0xFFFFFFFFu;
   return (uint32_t)floor((double)seed * 4294967295.0);
+}
+
+// The next ticket; none is left once a wait has been given up (what the other
+// nodes would be simulated from is not valid then).
+__device__ __forceinline__ int take_ticket(int* ctl) {
+  const int t = __hip_atomic_fetch_add(&ctl[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return ld_agent((const uint32_t*)&ctl[1]) ? 0x7FFFFFFF : t;
 }
 
 // Block-shared state of the current node.
@@ -272,7 +279,7 @@ __device__ __forceinline__ void gather_node(FlowArgs& P, int i, unsigned cell, i
       if (v >= P.nVar) continue;
       uint32_t b = bits[v];
       if (b == kPending && t != cell) {
-        b = wait_word(&wp[v], &P.ctl[1]);
+        b = wait_word(&wp[v], P.polls, &P.ctl[1]);
         waited = true;
       }
       val[v] = (b == kPending || b == kEmpty) ? NAN : __uint_as_float(b);
@@ -572,7 +579,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
     FlowArgs& P = *args();
     const int s0 = P.s[0], s1 = P.s[1], K = P.K, G = P.G;
     __syncthreads();  // the previous node's shared state is read no more
-    if (tid == 0) sh.tick = __hip_atomic_fetch_add(&P.ctl[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid == 0) sh.tick = take_ticket(P.ctl);
     __syncthreads();
     const int tick = __builtin_amdgcn_readfirstlane(sh.tick);
     const int q = tick / G, slice = tick - q * G;
@@ -909,8 +916,8 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
       if (tid < K) tk.push(best[tid]);
       for (int e = tid; e < (G - 1) * K; e += kThreads) {
         Cand64 c;
-        c.pos = (uint32_t)wait_word64(&sl[(long long)e * 2 + 1], &P.ctl[1]);
-        c.val = __longlong_as_double((long long)wait_word64(&sl[(long long)e * 2], &P.ctl[1]));
+        c.pos = (uint32_t)wait_word64(&sl[(long long)e * 2 + 1], P.polls, &P.ctl[1]);
+        c.val = __longlong_as_double((long long)wait_word64(&sl[(long long)e * 2], P.polls, &P.ctl[1]));
         c.h = tie_hash(seedbits, c.pos);
         if (c.pos != kNone) tk.push(c);
       }
@@ -983,7 +990,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
     const char* bits = reinterpret_cast<const char*>(P.bits);
     __syncthreads();  // the previous node's shared state is read no more
     if (tid == 0) {
-      sh.tick = __hip_atomic_fetch_add(&P.ctl[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.tick = take_ticket(P.ctl);
       sNt = 0;
     }
     __syncthreads();
@@ -1240,7 +1247,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
           }
       };
       if (tid < K) push((bestR[tid] >> 32 << 32) | sh.pos[tid]);
-      for (int e = tid; e < (G - 1) * K; e += kThreads) push(wait_word64(&sl[e], &P.ctl[1]));
+      for (int e = tid; e < (G - 1) * K; e += kThreads) push(wait_word64(&sl[e], P.polls, &P.ctl[1]));
       __syncthreads();  // bestR and sh.pos have been read
       block_best();
     }
@@ -1316,6 +1323,16 @@ static int flow_slices(const FlowPlan& F, long long S, int terms) {
   const long long pairs = S * terms;
   const long long per = F.count ? 1000000 : 160000;
   return (int)std::max<long long>(1, std::min<long long>(48, pairs / per));
+}
+
+// Polls of a wait: above any real one, which is what the nodes in flight take
+// one after another in the worst case, every slice summing all of its pairs at
+// 2 G pairs/s (a block alone reaches 10 and more). A poll takes at least its
+// s_sleep(2), 128 cycles: 53 ns at 2.4 GHz.
+static int flow_polls(const FlowPlan& F, long long S, int terms, int G, int cus) {
+  const double slice = (double)S * terms / G / 2e9;
+  const double nodes = std::min<double>(F.inFlight, 8.0 * cus / G + 1.0);  // at most 8 blocks per CU
+  return (int)std::min(2e9, (0.5 + nodes * slice) / 53e-9);
 }
 
 // Nodes after which FlowPlan::waveUs is compared with the time they took: the
@@ -1429,6 +1446,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   if (e != hipSuccess) return fail(QSMI_ERR_HIP, std::string("path loop set-up: ") + hipGetErrorString(e));
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, t->gpu) != hipSuccess || cus <= 0) cus = 256;
+  P.polls = t->tune.flowPolls > 0 ? t->tune.flowPolls : flow_polls(F, t->S, terms, P.G, cus);
   const int nv = R.n * R.nVar;
   const size_t lds = F.count ? (size_t)(2 * (((nv + 7) & ~7) + 8) + 2 * nv + 2 * R.n) * 4
                              : (size_t)(5 * (((nv + 7) & ~7) + 8) + R.nVar * kFlowQuant + 3 * nv + 2 * R.n) * 4;

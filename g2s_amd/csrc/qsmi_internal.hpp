@@ -28,6 +28,7 @@ struct ScanTune {
                            // (1024-grid scans on two lanes)
   int loopFlow = 1;        // 1: realisations that qualify run the data-flow path loop (qsmi_flow.hip); 0, or
                            // loopGraph: waves of FFT scans
+  int flowPolls = 0;       // polls after which the data-flow loop gives up a wait (0: above any real wait)
 };
 
 struct qsmi_ti {

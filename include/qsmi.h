@@ -107,6 +107,9 @@ int qsmi_ti_destroy(qsmi_ti* ti);
  *                 without transforms, where the request allows it (one TI,
  *                 not circular, no NaN, no learned proposal, record or -nV;
  *                 loop.graph 0): 0..1, default 1; 0: waves of transforms
+ *   "flow.polls"  polls after which that kernel gives up a wait and the path is
+ *                 simulated by waves of transforms instead (the same bytes):
+ *                 0..2^30, default 0: a bound above any real wait
  * Results do not depend on them up to the FP32 map error the exact selection
  * absorbs (pencil.npb, loop.graph, loop.flow: every choice gives the same bytes).
  * QSMI_ERR_ARG for an unknown key or a value out of range. */

@@ -116,6 +116,52 @@ def test_flow_slices_and_segments():
     assert flow["exact_nodes"] == waves["exact_nodes"]
 
 
+@pytest.mark.parametrize("kinds", [("cont",), ("3",), ("cont", "3")])
+def test_flow_gives_up(kinds):
+    """A wait that hits its bound (here the first poll that finds a value
+    missing) ends the loop; the wave loop simulates the path from its start."""
+    rng = np.random.default_rng(21)
+    dims, sdims = (150, 140), (30, 26)
+    ti = np.stack([_field(dims, rng, q) for q in kinds], 1).astype(np.float32)
+    di = np.full((int(np.prod(sdims)), len(kinds)), np.nan, np.float32)
+    types = [0 if q == "cont" else 1 for q in kinds]
+    out = []
+    try:
+        for key, value in (("flow.polls", 1), ("loop.flow", 0)):
+            g2s_amd.set_default_tuning(key, value)
+            out.append(g2s_amd.qs(ti, dims, di, sdims, types, 40, 1.5, 2, stage_timing=True))
+            g2s_amd.set_default_tuning("flow.polls", 0)
+    finally:
+        g2s_amd.set_default_tuning("loop.flow", 1)
+        g2s_amd.set_default_tuning("flow.polls", 0)
+    for a, b in zip(out[0][:2], out[1][:2]):
+        assert a.tobytes() == b.tobytes()
+    assert out[0][2]["gather_ms"] > 0.0
+
+
+def test_flow_gives_up_at_once():
+    """What is left of the path after a given-up wait is not simulated: on an
+    image where the data-flow loop takes longer than the waves (white noise,
+    250 neighbours, 10 best), the run costs little more than the waves alone.
+    Half of their time is room for the first nodes and the timer; the rest of
+    the path would take more than all of it."""
+    rng = np.random.default_rng(22)
+    dims, sdims = (1000, 1000), (100, 100)
+    ti = rng.standard_normal(dims[0] * dims[1]).astype(np.float32)
+    di = np.full(sdims[0] * sdims[1], np.nan, np.float32)
+    ms = {}
+    try:
+        for name, key, value in (("warm", "loop.flow", 0), ("waves", "loop.flow", 0), ("given up", "flow.polls", 1)):
+            g2s_amd.set_default_tuning("loop.flow", 1)
+            g2s_amd.set_default_tuning(key, value)
+            ms[name] = g2s_amd.qs(ti, dims, di, sdims, [0], 250, 10.0, 6)[2]["path_loop_ms"]
+            print(f"data-flow loop: {name} {ms[name]:.0f} ms", flush=True)
+    finally:
+        g2s_amd.set_default_tuning("loop.flow", 1)
+        g2s_amd.set_default_tuning("flow.polls", 0)
+    assert ms["given up"] < 1.5 * ms["waves"]
+
+
 def test_flow_hands_over_to_waves():
     """White noise on the 1024 grid: the first nodes take longer than the wave
     loop's, which starts over (or the data-flow loop goes on: same bytes)."""
