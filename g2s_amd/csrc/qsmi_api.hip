@@ -614,6 +614,7 @@ const TuneKey kTuneKeys[] = {
     {"fft.lognv_max", &ScanTune::lognvMax, 0, 6},
     {"loop.graph", &ScanTune::loopGraph, 0, 1},
     {"loop.flow", &ScanTune::loopFlow, 0, 1},
+    {"flow.nodes", &ScanTune::flowNodes, 0, 1 << 30},
     {"flow.polls", &ScanTune::flowPolls, 0, 1 << 30},
 };
 const TuneKey* find_tune_key(const char* key) {

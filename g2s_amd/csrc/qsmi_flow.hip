@@ -72,6 +72,7 @@ constexpr int kThreads = 256, kWaves = kThreads / 64;
 constexpr int kTileX = 16, kTileY = 4, kPair = 2, kRun = 16;
 constexpr int kStep = 8;        // terms between two looks at the bound
 constexpr int kWaveList = 256;  // kept positions of a wavefront before they are scored
+constexpr int kFlowStats = 7;
 constexpr int kSources = 32;    // neighbours whose source positions seed the bound
 
 struct FlowParams {
@@ -105,7 +106,7 @@ struct FlowParams {
   int* ctl;           // [0] ticket (kNoTicket and above: none left), [1] a wait was given up
   int polls;          // polls after which a wait is given up
   unsigned long long* slots;
-  unsigned long long* stats;
+  unsigned long long* stats;  // [kFlowStats]: nodes, positions scored, 0, flushes; tiles, their steps, without the bound
   int node0, nNodes;
 };
 
@@ -547,7 +548,9 @@ __device__ __forceinline__ float uniform(float v) {
 
 // FORM 0: continuous, every weight 1 or 0 (no value); 1: continuous; 2: with
 // categorical variables. NV: 1 for one variable, else at least their number.
-template <int FORM, int NV, int KT>
+// COUNT: tiles and steps are counted (a scalar more in the tile loop, 1 % of the
+// scan, so only the segments that are judged by them do).
+template <int FORM, int NV, int KT, bool COUNT>
 __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_flow_direct(FlowParams kernArgs) {
   constexpr bool MIXED = FORM == 2;
   extern __shared__ __align__(16) char dyn[];
@@ -577,6 +580,8 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
   __builtin_amdgcn_s_setprio(3);
   for (int t = tid; t < nVar * kFlowQuant; t += kThreads) quant[t] = P0.quant[t];  // first read after a barrier
   unsigned long long nScored = 0, nNodesDone = 0, nFlush = 0;
+  // tiles of the block's nodes, their steps without the bound, and the steps this wavefront took
+  unsigned long long nTiles = 0, nFull = 0, nSteps = 0;
   for (;;) {
     FlowArgs& P = *args();
     const int s0 = P.s[0], s1 = P.s[1], K = P.K, G = P.G;
@@ -720,6 +725,10 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
     tk.init();
     const int NX = (n[0] + kTileX * kPair - 1) / (kTileX * kPair), NY = (n[1] + kTileY - 1) / kTileY;
     const int units = box ? NX * NY * n[2] : 0;
+    if (COUNT && slice == G - 1) {
+      nTiles += (unsigned)units;
+      nFull += (unsigned long long)units * ((unsigned)(Tn + kStep - 1) / kStep);
+    }
     // a node's dependents wait for everything but the scan's share of the
     // other nodes: the scan yields to the short phases around it
     __builtin_amdgcn_s_setprio(0);
@@ -739,6 +748,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
         fw[e] = FORM == 0 ? 1.f : uniform(tW[e]);
         fc[e] = MIXED ? uniform(tC[e]) : 0.f;
       }
+      unsigned terms = 0;  // of this wavefront's units, in whole steps
       int k = 0;  // the slice's units, handed out to its wavefronts one by one
       if (lane == 0) k = atomicAdd(&sh.unit, 1);
       for (;;) {
@@ -779,7 +789,8 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
         }
         // wave-uniform: a position can still be within the limit
         bool on = __any(fminf(acc[0], acc[1]) <= lim);
-        for (int t = kStep; t < Tn && on; t += kStep) {
+        int t = kStep;
+        for (; t < Tn && on; t += kStep) {
           int o[kStep];
           float x[kStep], w[kStep], c[kStep];
 #pragma unroll
@@ -798,6 +809,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
           }
           on = __any(fminf(acc[0], acc[1]) <= lim);
         }
+        if (COUNT) terms += (unsigned)t;
         if (!on) continue;
 #pragma unroll
         for (int r = 0; r < kPair; ++r) {
@@ -847,6 +859,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
           lim = cost_limit(thr, W, Tn);
         }
       }
+      if (COUNT) nSteps += terms / kStep;
     }
     __builtin_amdgcn_s_setprio(3);
     // the slice's bound: every wavefront's K-th cost holds for all
@@ -934,6 +947,11 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
   if (lane == 0 && nScored) atomicAdd(&P0.stats[1], nScored);
   if (lane == 0 && nFlush) atomicAdd(&P0.stats[3], nFlush);
   if (tid == 0 && nNodesDone) atomicAdd(&P0.stats[0], nNodesDone);
+  if (COUNT && lane == 0 && nSteps) atomicAdd(&P0.stats[5], nSteps);
+  if (COUNT && tid == 0 && nTiles) {
+    atomicAdd(&P0.stats[4], nTiles);
+    atomicAdd(&P0.stats[6], nFull);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1342,13 +1360,65 @@ static int flow_polls(const FlowPlan& F, long long S, int terms, int G, int cus)
   return (int)std::min(2e9, (0.5 + nodes * slice) / 53e-9);
 }
 
-// Nodes after which FlowPlan::waveUs is compared with the time they took: the
-// first and slowest ones, whose neighbours are far.
-constexpr int kFlowJudge = 65536;
+// The direct scan against the waves, for what is left of a path. The waves'
+// transforms cost the same for every image, the direct scan less the sooner
+// its bound rules a position out, so the choice is made between segments from
+// the tiles and steps that the kernel counted (not from a clock: the same
+// request takes the same route under any load).
+//
+// A chip full of nodes takes kTileUs a tile and stepUs a step; where a level
+// has few nodes, it takes a node from its last neighbour's value to its own:
+// 50 us, 0.2 us a term (gather, order, merge) and, one after another, the
+// steps of one of the node's 4 G wavefronts, 0.45 us each. Measured against
+// that, us a node (K <= 2, white noise unless said):
+//   1000 x 1000, 1 variable, n 20 / 80 / 250: 2.0 / 4.9 / 16.4 (13.2 K / 40.7 K / 139 K steps)
+//   the same, n 80, correlation length 20 / 8: 1.8-3.0 / 2.1-3.7 (11-24 K / 14-30 K steps)
+//   1000 x 1000, 2 variables, n 60: 9.9 (63.9 K); with 4 classes, n 80: 18.6 (129 K), smooth 6.3 (41 K)
+//   levels of few nodes, us a level: 530 (1000 x 1000, n 250, 139 K steps), 800 (two variables), 316 and 805
+//   (1500 x 1500, n 80 and 250, 84 K and 289 K), 154 and 175 (120 x 120 and 250 x 250, n 500)
+// More than two best positions cost registers and list flushes: 0.135 ns a
+// step instead of 0.105 at 3, 0.25 at 10 (two variables 0.145, 0.19, 0.7).
+constexpr double kTileUs = 0.88e-4;
+struct FlowCost {
+  double nodeUs, levelUs;
+};
+static FlowCost flow_cost(double tiles, double steps, int terms, int nVar, int K, int G) {
+  const double one = nVar == 1 ? 1.05e-4 : 1.45e-4;
+  const double stepUs = K <= 2 ? one : nVar == 1 ? (K <= 4 ? 1.35e-4 : 2.5e-4) : (K <= 4 ? 1.9e-4 : 7.0e-4);
+  return {tiles * kTileUs + steps * stepUs, 50.0 + 0.2 * terms + 0.45 * (stepUs / one) * steps / (kWaves * G)};
+}
 
-int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, bool* gaveUp) {
+// The nodes of R's order from `first` on. A level's nodes wait for the one
+// before; at most inFlight of them run at a time.
+static double flow_path_us(const FlowPlan& F, const ResidentLoop& R, size_t first, const FlowCost& c) {
+  double us = 0.0;
+  const size_t nW = R.waveLevel.size();
+  for (size_t w = 0; w < nW;) {
+    const int level = R.waveLevel[w];
+    size_t b = (size_t)R.waveStart[w];
+    while (w < nW && R.waveLevel[w] == level) ++w;
+    const size_t e = (size_t)R.waveStart[w];
+    if (e <= first) continue;
+    const double m = (double)(e - std::max(b, first));
+    us += std::max(m * c.nodeUs, std::ceil(m / F.inFlight) * c.levelUs);
+  }
+  return us;
+}
+static double wave_path_us(const FlowPlan& F, const ResidentLoop& R, size_t first) {
+  double us = F.waveSetupUs;
+  for (size_t w = 0; w < R.waveLevel.size(); ++w) {
+    const size_t b = std::max((size_t)R.waveStart[w], first), e = (size_t)R.waveStart[w + 1];
+    if (e > b) us += F.waveUs + (double)(e - b) * F.waveNodeUs;
+  }
+  return us;
+}
+constexpr double kHandOver = 1.05;  // the models are good to some 10 %; a segment decides anew
+
+int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, size_t* doneOut,
+             bool* gaveUp) {
   hipStream_t st = t->stream;
   *gaveUp = false;
+  *doneOut = 0;
   const size_t nPath = (size_t)F.nPath;
   FlowParams P;
   memset(&P, 0, sizeof(P));
@@ -1419,7 +1489,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   };
   P.work = (uint32_t*)alloc(SD * R.nVar * sizeof(uint32_t));
   P.ctl = (int*)alloc(2 * sizeof(int));
-  P.stats = (unsigned long long*)alloc(4 * sizeof(unsigned long long));
+  P.stats = (unsigned long long*)alloc(kFlowStats * sizeof(unsigned long long));
   P.slots = (unsigned long long*)alloc(slotWords * sizeof(unsigned long long));
   float* planes = F.count ? nullptr : (float*)alloc((size_t)R.nVar * t->S * sizeof(float));
   uint32_t* bits = F.count ? (uint32_t*)alloc(((size_t)(F.nClasses + 1) * P.planeWords + 4) * sizeof(uint32_t)) : nullptr;
@@ -1435,7 +1505,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
     P.quant = dq;
   }
   if (e == hipSuccess) e = hipMemsetAsync(P.ctl, 0, 2 * sizeof(int), st);
-  if (e == hipSuccess) e = hipMemsetAsync(P.stats, 0, 4 * sizeof(unsigned long long), st);
+  if (e == hipSuccess) e = hipMemsetAsync(P.stats, 0, kFlowStats * sizeof(unsigned long long), st);
   const long long words = (long long)SD * R.nVar;
   hipLaunchKernelGGL(k_flow_grid, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, R.dDi, P.work, words);
   if (F.count && e == hipSuccess)
@@ -1465,38 +1535,70 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   double ms = 0.0;
   const auto begun = std::chrono::steady_clock::now();
   auto told = begun;
-  bool slow = false, judged = !(F.waveUs > 0.0);
-  for (size_t b = 0; b < nPath && e == hipSuccess && !slow; b += seg) {
+  // Whether the waves may be the faster ones: not if the scan is ahead of them
+  // with every step of every tile. Otherwise the first segments end after n
+  // nodes (whose neighbour lists are still filling), four times that, ... and
+  // are judged each; from 65536 nodes on, the 8192 after every 65536.
+  bool slow = false;
+  bool judge = F.waveNodeUs > 0.0;
+  const double maxSteps = (terms + kStep - 1) / kStep;
+  if (judge) {
+    const double tiles = (double)((t->s[0] + kTileX * kPair - 1) / (kTileX * kPair)) * ((t->s[1] + kTileY - 1) / kTileY) *
+                         t->s[2];
+    judge = flow_path_us(F, R, 0, flow_cost(tiles, tiles * maxSteps, terms, R.nVar, P.K, P.G)) >
+            kHandOver * wave_path_us(F, R, 0);
+  }
+  size_t countFrom = judge ? 0 : nPath, verdict = (size_t)std::max(64, R.n);  // nodes counted, then judged
+  unsigned long long seen[kFlowStats] = {};
+  size_t done = 0;
+  const size_t stop = t->tune.flowNodes > 0 ? std::min(nPath, (size_t)t->tune.flowNodes) : nPath;
+  for (size_t b = 0; b < stop && e == hipSuccess && !slow; b = done) {
     P.node0 = (int)b;
-    P.nNodes = (int)std::min(seg, nPath - b);
+    const bool counted = b >= countFrom;
+    P.nNodes = (int)std::min({seg, stop - b, (counted ? verdict : countFrom) - b});
     if (b) hipLaunchKernelGGL(k_flow_next, dim3(1), dim3(1), 0, st, P.ctl);
     if (e == hipSuccess && slotWords) e = hipMemsetAsync(P.slots, 0xFF, slotWords * sizeof(unsigned long long), st);
     if (ev[0] && ev[1]) (void)hipEventRecord(ev[0], st);
     const int maxBlocks = (int)std::min<long long>((long long)P.nNodes * P.G, (long long)F.inFlight * P.G);
-#define QSMI_FLOW(KT_)                                                                                       \
-  e = F.count ? (terms < 128 ? (R.nVar == 1 ? launch_persistent(k_flow_count<7, 1, KT_>, P, lds, maxBlocks, cus, st)   \
-                                            : launch_persistent(k_flow_count<7, 8, KT_>, P, lds, maxBlocks, cus, st))  \
-                             : launch_persistent(k_flow_count<10, 8, KT_>, P, lds, maxBlocks, cus, st))                \
-      : F.mixed ? (R.nVar <= 2 ? launch_persistent(k_flow_direct<2, 2, KT_>, P, lds, maxBlocks, cus, st)     \
-                               : launch_persistent(k_flow_direct<2, 8, KT_>, P, lds, maxBlocks, cus, st))    \
-      : R.nVar > 1 ? launch_persistent(k_flow_direct<1, 8, KT_>, P, lds, maxBlocks, cus, st)                 \
-      : F.unitW    ? launch_persistent(k_flow_direct<0, 1, KT_>, P, lds, maxBlocks, cus, st)                 \
-                   : launch_persistent(k_flow_direct<1, 1, KT_>, P, lds, maxBlocks, cus, st)
+#define QSMI_COUNT(NP_, NV_, KT_) launch_persistent(k_flow_count<NP_, NV_, KT_>, P, lds, maxBlocks, cus, st)
+#define QSMI_DIRECT(FORM_, NV_, KT_)                                                              \
+  (counted ? launch_persistent(k_flow_direct<FORM_, NV_, KT_, true>, P, lds, maxBlocks, cus, st) \
+           : launch_persistent(k_flow_direct<FORM_, NV_, KT_, false>, P, lds, maxBlocks, cus, st))
+#define QSMI_FLOW(KT_)                                                                           \
+  e = F.count ? (terms >= 128  ? QSMI_COUNT(10, 8, KT_)                                          \
+                 : R.nVar == 1 ? QSMI_COUNT(7, 1, KT_)                                           \
+                               : QSMI_COUNT(7, 8, KT_))                                          \
+      : F.mixed    ? (R.nVar <= 2 ? QSMI_DIRECT(2, 2, KT_) : QSMI_DIRECT(2, 8, KT_))             \
+      : R.nVar > 1 ? QSMI_DIRECT(1, 8, KT_)                                                      \
+      : F.unitW    ? QSMI_DIRECT(0, 1, KT_)                                                      \
+                   : QSMI_DIRECT(1, 1, KT_)
     if (e != hipSuccess) break;
     if (P.K <= 2) QSMI_FLOW(2);
     else if (P.K <= 4) QSMI_FLOW(4);
     else QSMI_FLOW(16);
 #undef QSMI_FLOW
+#undef QSMI_DIRECT
+#undef QSMI_COUNT
     if (ev[0] && ev[1]) {
       (void)hipEventRecord(ev[1], st);
       float one = 0.f;
       if (hipEventSynchronize(ev[1]) == hipSuccess && hipEventElapsedTime(&one, ev[0], ev[1]) == hipSuccess) ms += one;
     }
-    const size_t done = b + (size_t)P.nNodes;
-    if (!judged && done >= (size_t)kFlowJudge && hipStreamSynchronize(st) == hipSuccess) {
-      judged = true;
-      slow = std::chrono::duration<double, std::micro>(std::chrono::steady_clock::now() - begun).count() >
-             F.waveUs * (double)done;
+    done = b + (size_t)P.nNodes;
+    if (counted && done == verdict && done < nPath) {
+      unsigned long long sv[kFlowStats];
+      e = hipStreamSynchronize(st);
+      if (e == hipSuccess) e = hipMemcpy(sv, P.stats, sizeof(sv), hipMemcpyDeviceToHost);
+      if (e != hipSuccess) break;
+      const double nodes = (double)(done - countFrom), tiles = (double)(sv[4] - seen[4]) / nodes, full = (double)(sv[6] - seen[6]) / nodes;
+      double steps = (double)(sv[5] - seen[5]) / nodes;
+      // the first lists are short: what comes after the first step grows with them
+      if (countFrom == 0 && full > tiles) steps = tiles + (steps - tiles) * std::max(1.0, tiles * (maxSteps - 1.0) / (full - tiles));
+      slow = flow_path_us(F, R, done, flow_cost(tiles, steps, terms, R.nVar, P.K, P.G)) >
+             kHandOver * wave_path_us(F, R, done);
+      memcpy(seen, sv, sizeof(sv));
+      countFrom = done < 65536 ? done : done + 65536;
+      verdict = done < 65536 ? 4 * done : countFrom + 8192;
     }
     if (R.progressSec > 0 && hipStreamSynchronize(st) == hipSuccess) {
       const auto now = std::chrono::steady_clock::now();
@@ -1513,13 +1615,14 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   hipLaunchKernelGGL(k_flow_finish, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, R.dDi, P.work, words);
   if (e == hipSuccess) e = hipGetLastError();
   int ctl[2] = {0, 0};
-  unsigned long long sv[4] = {0, 0, 0, 0};
+  unsigned long long sv[kFlowStats] = {};
   const hipError_t es = hipStreamSynchronize(st);
   if (e == hipSuccess) e = es;
   if (e == hipSuccess) e = hipMemcpy(ctl, P.ctl, sizeof(ctl), hipMemcpyDeviceToHost);
   if (e == hipSuccess) e = hipMemcpy(sv, P.stats, sizeof(sv), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return fail(QSMI_ERR_HIP, std::string("path loop: ") + hipGetErrorString(e));
-  *gaveUp = ctl[1] != 0 || slow;
+  *gaveUp = ctl[1] != 0;
+  *doneOut = done;
   *kernelMs = ms;
   for (int q = 0; q < 4; ++q) stats[q] = (long long)sv[q];
   return QSMI_OK;

@@ -19,13 +19,17 @@ struct FlowPlan {
   float rare[kFlowMaxCat] = {};                // per class: 1 - its share of the TI
   int inFlight = 1 << 20;  // path nodes simulated at the same time, at most
   int segment = 65536;     // path nodes per launch
-  double waveUs = 0.0;     // microseconds a node above which the wave loop is the faster one (0: never)
+  // what the wave loop takes, microseconds: a wave, a node, its spectra and
+  // buffers (waveNodeUs 0: the path is never handed over to it)
+  double waveUs = 0.0, waveNodeUs = 0.0, waveSetupUs = 0.0;
 };
 
 // Simulates the path (R's neighbour lists, grid and tables on the device).
 // stats: exact-selection nodes, rescored positions, 0, list flushes.
-// gaveUp: a wait hit its bound, or the first nodes took longer than waveUs
-// each; the grid is not usable then.
-int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, bool* gaveUp);
+// done: nodes of R's order that are simulated, in the grid and the index image;
+// the rest, if any, is faster by waves.
+// gaveUp: a wait hit its bound; the grid is not usable then.
+int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kernelMs, long long* stats, size_t* done,
+             bool* gaveUp);
 
 }  // namespace qsmi

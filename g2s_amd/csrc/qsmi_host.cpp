@@ -442,6 +442,31 @@ bool plan_flow(const qsmi_qs_request* rq, const ScanTune& tune, int D, const flo
   return true;
 }
 
+// What the wave loop takes, for the choice between it and the data-flow loop
+// (V sub-images, n neighbours, K best; microseconds). Fitted to two paths each
+// of few and of many nodes a wave; us a wave + us a node measured:
+//   1024 x 1024 grid, V 2: 125 + 3.0 (n 20), 121 + 3.2-3.6 (80), 148 + 5.1-6.4 (250), 188 + 12.8 (500);
+//                     V 4: 176 + 5.3 (60), 310 + 13.7 (250); V 6: 214 + 6.3 (60), 395 + 19.4 (250)
+//   own grids, ps a cell and node: 2-D 26-31 (V 2), 38 (4), 46 (6) with waves of 84-404, 144-374, 170 us;
+//                     3-D, V 2: 22-24 (n 30), 27-30 (100), 56-79 (300) with 103-383 us; n 100: 51 (V 4), 69 (6)
+// K above 2 costs about a microsecond a node each (1000 x 1000: 8.6 at 10).
+// Spectra and buffers: 13 ms on 1000 x 1000 with V 2, 20 with V 4, 1.1 on 250 x 250.
+void wave_cost(const qsmi_ti* ti, int V, int n, int K, qsmi::FlowPlan* F) {
+  const double more = std::max(0, n - 80);
+  if (ti->w1k) {
+    F->waveUs = 70.0 + 24.5 * V + 0.2 * (V - 1) * std::max(0, n - 60);
+    F->waveNodeUs = 1.2 + 0.9 * V + 0.012 * (V - 1) * more;
+  } else if (ti->D < 3) {
+    F->waveUs = 50.0 + 17.0 * V + 0.2 * V * n;
+    F->waveNodeUs = (18.0 + 4.8 * V) * 1e-6 * (double)ti->N;
+  } else {
+    F->waveUs = 50.0 + 17.0 * V + 0.35 * V * n;
+    F->waveNodeUs = (12.0 + V * (4.5 + 0.035 * n)) * 1e-6 * (double)ti->N;
+  }
+  F->waveNodeUs += std::max(0, K - 2);
+  F->waveSetupUs = 1000.0 + 0.0065 * V * (double)ti->S;
+}
+
 int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   using clk = std::chrono::steady_clock;
   if (!rq || !rs || !rs->simulation || !rs->index) return hfail(QSMI_ERR_ARG, "null argument");
@@ -693,15 +718,18 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   // device: TI spectra + scan engine
   std::vector<qsmi_ti*> xti;
   std::vector<qsmi_device*> xdev;
-  if (!useFlow) {
+  auto scan_device = [&]() -> int {
     std::vector<float> sub((size_t)nSub * S);
     if (cross)
       qsmi_ti_subimages_x(D, s, nVar, rq->varTypes, tiData, sub.data());
     else
       qsmi_ti_subimages(D, s, nVar, rq->varTypes, tiIn, ncat.data(), catvals.data(), sub.data());
-    rc = qsmi_ti_create(rq->gpu, D, s, nullptr, nSub, sub.data(), &ti);
-    if (rc) return rc;
-    rc = qsmi_device_create(ti, alpha, rq->circularTI ? 1 : 0, &dev);
+    const int e = qsmi_ti_create(rq->gpu, D, s, nullptr, nSub, sub.data(), &ti);
+    return e ? e : qsmi_device_create(ti, alpha, rq->circularTI ? 1 : 0, &dev);
+  };
+  if (!useFlow) {
+    rc = scan_device();
+    if (rc && !ti) return rc;
   }
   if (!rc && cross) rc = qsmi::set_cross(dev, alphaX, centreOk.data());
   // the other TIs: spectra and a device each
@@ -987,21 +1015,10 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
         flow.inFlight = rq->waveSize;
         flow.segment = (int)std::min<long long>(flow.segment, 64ll * rq->waveSize);
       }
-      // The wave loop's transforms cost the same for every image, the direct
-      // scan less the sooner its bound rules a position out. On the 1024 x
-      // 1024 grid, the one where the transforms come close, 80 neighbours and
-      // full waves take 3.25 us a node (250 neighbours 5.1) and the direct
-      // scan of a 1000 x 1000 image 2.9 (correlation length 20), 3.5 (8), 4.3
-      // (3) and 5.0 (white noise); its first 65536 nodes take 3.1, 4.3, 5.9
-      // and 6.2. Starting over pays above 4.6, where the path is long enough
-      // for that and its levels wide enough to fill waves: noise then takes
-      // 3.24 s + 0.4 s instead of 5.0. On every other grid the direct scan
-      // stays ahead in noise too (500 x 500: 1.8 us a node against 3.3).
-      if (D == 2 && ti->w1k && nVar == 1 && !flow.count && nPath >= 4 * 65536 && flow.inFlight >= 256 &&
-          S > 600 * 1000)
-        flow.waveUs = 4.6 + 0.011 * std::max(0, nMax - 80);
+      if (!flow.count) wave_cost(ti, nSub, nMax, (int)std::ceil(kMax), &flow);
+      size_t done = 0;
       bool gaveUp = false;
-      rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &gaveUp);
+      rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &done, &gaveUp);
       scanned = (long long)nPath;
       waves = (int)R.waveLevel.size();
       if (!rc && gaveUp) {  // the wave loop, from the start
@@ -1016,6 +1033,27 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
           rs->phaseMs[3] += lost;
         }
         return rc;
+      }
+      if (!rc && done < nPath) {  // the rest by waves
+        qsmi_ti_destroy(ti);
+        ti = nullptr;
+        rc = scan_device();
+        if (!rc) {
+          qsmi_set_tie_quantum(dev, quantum);
+          size_t w = 0;
+          while ((size_t)R.waveStart[w + 1] <= done) ++w;
+          R.waveStart.erase(R.waveStart.begin(), R.waveStart.begin() + w);
+          R.waveLevel.erase(R.waveLevel.begin(), R.waveLevel.begin() + w);
+          R.waveStart[0] = (int)done;
+          double ms[4] = {0, 0, 0, 0};
+          long long band[4] = {0, 0, 0, 0}, sc = 0;
+          int wv = 0;
+          rc = qsmi::run_resident_waves(dev, R, ms, &sc, &wv, band);
+          for (int q = 0; q < 4; ++q) {
+            stageMs[q] += ms[q];
+            bandStats[q] += band[q];
+          }
+        }
       }
     } else {
       rc = qsmi::run_resident_waves(dev, R, stageMs, &scanned, &waves, bandStats);

@@ -28,6 +28,7 @@ struct ScanTune {
                            // (1024-grid scans on two lanes)
   int loopFlow = 1;        // 1: realisations that qualify run the data-flow path loop (qsmi_flow.hip); 0, or
                            // loopGraph: waves of FFT scans
+  int flowNodes = 0;       // nodes that the data-flow loop leaves to the wave loop after (0: where that is the faster)
   int flowPolls = 0;       // polls after which the data-flow loop gives up a wait (0: above any real wait)
 };
 

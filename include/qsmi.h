@@ -106,7 +106,11 @@ int qsmi_ti_destroy(qsmi_ti* ti);
  *                 simulates every node as soon as its neighbours hold values,
  *                 without transforms, where the request allows it (one TI,
  *                 not circular, no NaN, no learned proposal, record or -nV;
- *                 loop.graph 0): 0..1, default 1; 0: waves of transforms
+ *                 loop.graph 0), and by waves of transforms from where those
+ *                 are the faster: 0..1, default 1; 0: waves from the start
+ *   "flow.nodes"  path nodes after which that kernel hands over to waves (the
+ *                 same bytes): 0..2^30, default 0: where the work that it
+ *                 counts says so
  *   "flow.polls"  polls after which that kernel gives up a wait and the path is
  *                 simulated by waves of transforms instead (the same bytes):
  *                 0..2^30, default 0: a bound above any real wait

@@ -6,8 +6,6 @@ form that the data-flow loop takes: 1-3 dimensions, extents around the tile
 and word edges (16, 32, 64), list lengths, weights, given and partially given
 cells, images of n and k, several kernels, wrapping grids and images whose
 best positions tie by the thousand."""
-import sys
-
 import numpy as np
 import pytest
 
@@ -69,11 +67,9 @@ CASES = [
 ]
 
 
-@pytest.mark.parametrize("case", range(len(CASES)))
-def test_flow_equals_waves(case):
+def _request(case):
     kinds, dims, sdims, n, k, x = CASES[case]
     print(f"data-flow loop: case {case} {CASES[case]}", flush=True)
-    sys.stdout.flush()
     rng = np.random.default_rng(100 + case)
     types = [0 if q in ("cont", "flat", "steps") else 1 for q in kinds]
     ti = np.stack([_field(dims, rng, q) for q in kinds], 1).astype(np.float32)
@@ -102,7 +98,29 @@ def test_flow_equals_waves(case):
         sizes = [kd, [9, 11]]
         kw.update(kernels=[np.ones(int(np.prod(s)), np.float32) for s in sizes], kernels_dims=sizes,
                   kernel_index_image=rng.integers(0, 2, cells).astype(np.float32))
-    _both(ti, dims, di, sdims, types, n, k, 5 + case, **kw)
+    return (ti, dims, di, sdims, types, n, k, 5 + case), kw
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_flow_equals_waves(case):
+    args, kw = _request(case)
+    _both(*args, **kw)
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_flow_then_waves(case):
+    """The path handed over in the middle, at a place that cuts a level."""
+    args, kw = _request(case)
+    try:
+        g2s_amd.set_default_tuning("flow.nodes", int(np.prod(CASES[case][2])) // 3)
+        a = g2s_amd.qs(*args, stage_timing=True, **kw)
+        g2s_amd.set_default_tuning("loop.flow", 0)
+        b = g2s_amd.qs(*args, **kw)
+    finally:
+        g2s_amd.set_default_tuning("flow.nodes", 0)
+        g2s_amd.set_default_tuning("loop.flow", 1)
+    assert a[0].tobytes() == b[0].tobytes() and a[1].tobytes() == b[1].tobytes()
+    assert a[2]["gather_ms"] > 0.0 and a[2]["waves"] == b[2]["waves"]
 
 
 def test_flow_slices_and_segments():
@@ -162,18 +180,28 @@ def test_flow_gives_up_at_once():
     assert ms["given up"] < 1.5 * ms["waves"]
 
 
-def test_flow_hands_over_to_waves():
-    """White noise on the 1024 grid: the first nodes take longer than the wave
-    loop's, which starts over (or the data-flow loop goes on: same bytes)."""
+@pytest.mark.parametrize("kinds,n,sdims,over", [
+    (("noise",), 80, (530, 500), True),
+    (("noise",), 250, (120, 120), True),
+    (("noise", "noise"), 60, (100, 100), True),
+    (("cont",), 80, (150, 150), False),
+])
+def test_flow_hands_over_to_waves(kinds, n, sdims, over):
+    """1000 x 1000 images: white noise, where the wave loop takes over the rest
+    of the path, and a smooth image, where it does not."""
     rng = np.random.default_rng(8)
-    dims, sdims = (1000, 1000), (530, 500)
-    ti = rng.standard_normal(dims[0] * dims[1]).astype(np.float32)
-    di = np.full(sdims[0] * sdims[1], np.nan, np.float32)
+    dims = (1000, 1000)
+    ti = [rng.standard_normal(dims[0] * dims[1]) if q == "noise" else _field(dims, rng, q) for q in kinds]
+    ti = np.stack(ti, 1).astype(np.float32)
+    di = np.full((sdims[0] * sdims[1], len(kinds)), np.nan, np.float32)
     out = []
     try:
         for flow in (1, 0):
             g2s_amd.set_default_tuning("loop.flow", flow)
-            out.append(g2s_amd.qs(ti, dims, di, sdims, [0], 80, 1.5, 6))
+            out.append(g2s_amd.qs(ti, dims, di, sdims, [0] * len(kinds), n, 1.5, 6, stage_timing=True))
     finally:
         g2s_amd.set_default_tuning("loop.flow", 1)
     assert out[0][0].tobytes() == out[1][0].tobytes() and out[0][1].tobytes() == out[1][1].tobytes()
+    assert out[0][2]["exact_nodes"] == out[1][2]["exact_nodes"]
+    # only the wave loop has a gather stage; less of it where it came in later
+    assert (0.0 < out[0][2]["gather_ms"] < out[1][2]["gather_ms"]) if over else out[0][2]["gather_ms"] == 0.0
