@@ -373,12 +373,14 @@ namespace {
 
 // How the realisation qualifies for the data-flow path loop, or false. Its
 // direct form selects exactly as the exact selection does and its count form
-// as the tie quantum does when the quantum divides the weight, so only
-// requests whose wave loop would do the same qualify. tiIn, di: finite, and
-// small enough that no sum of squares overflows.
+// as the tie quantum does when the quantum divides the weight and is no finer
+// than the default one (minQuantum: half of a finer one can be less than the
+// FP32 map's error, and the wave loop then splits ties that counts keep), so
+// only requests whose wave loop would do the same qualify. tiIn, di: finite,
+// and small enough that no sum of squares overflows.
 bool plan_flow(const qsmi_qs_request* rq, const ScanTune& tune, int D, const float* tiIn, size_t S, size_t SD, int nMax,
                const std::vector<int>& ncat, const std::vector<float>& catvals, const std::vector<float>& kernels,
-               int nExp, float quantum, qsmi::FlowPlan* F) {
+               int nExp, float quantum, float minQuantum, qsmi::FlowPlan* F) {
   const int nVar = rq->nVar;
   if (!tune.loopFlow || tune.loopGraph || rq->nTI > 1 || rq->circularTI || rq->lp || rq->recordCap > 0 || rq->noVerbatim)
     return false;
@@ -413,7 +415,7 @@ bool plan_flow(const qsmi_qs_request* rq, const ScanTune& tune, int D, const flo
   F->mixed = anyCat;
   if (F->count && quantum > 0.f) {
     const float r = w0 / quantum;
-    if (!(r >= 2.f && r <= 65536.f && r == std::floor(r) && r * quantum == w0)) return false;
+    if (!(quantum >= minQuantum && r >= 2.f && r <= 65536.f && r == std::floor(r) && r * quantum == w0)) return false;
   } else if (quantum != 0.f) {
     return false;
   }
@@ -690,21 +692,19 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   const size_t nPath = SD - begin;
   bool anyCont = false;
   for (int v = 0; v < nVar; ++v) anyCont |= rq->varTypes[v] == 0;
-  float quantum = rq->tieQuantum;
-  if (quantum < 0.f) {
-    quantum = 0.f;
-    if (!anyCont && maxw > 0.f) {
-      int e2 = (int)std::ceil(std::log2((double)nMax * (double)maxw));
-      quantum = std::ldexp(1.f, e2 - 16);
-    }
+  float defaultQuantum = 0.f;
+  if (!anyCont && maxw > 0.f) {
+    int e2 = (int)std::ceil(std::log2((double)nMax * (double)maxw));
+    defaultQuantum = std::ldexp(1.f, e2 - 16);
   }
+  const float quantum = rq->tieQuantum < 0.f ? defaultQuantum : rq->tieQuantum;
   // the data-flow path loop needs neither spectra nor a scan device
   qsmi_ti* ti = nullptr;
   qsmi_device* dev = nullptr;
   qsmi::FlowPlan flow;
   bool useFlow = allowFlow && !cross &&
                  plan_flow(rq, qsmi::default_tune(), D, tiIn, S, SD, nMax, ncat, catvals, ker.data, nExp, quantum,
-                           &flow);
+                           defaultQuantum, &flow);
   int rc = QSMI_OK;
   if (useFlow) {
     rc = qsmi::ti_create(rq->gpu, D, s, nullptr, nSub, nullptr, &ti);

@@ -134,6 +134,28 @@ def test_flow_slices_and_segments():
     assert flow["exact_nodes"] == waves["exact_nodes"]
 
 
+@pytest.mark.parametrize("n,default,finer", [(50, -10, 0), (50, -10, 1), (300, -7, 9)])
+def test_flow_tie_quantum(n, default, finer):
+    """A tie quantum finer than the default (2^default for n neighbours of
+    weight 1) may be less than twice the FP32 map's error (2^-16 is less than
+    the spacing of FP32 numbers at 300): the wave loop's selection is what the
+    request gets then."""
+    rng = np.random.default_rng(31)
+    dims, sdims = (250, 250), (40, 36)
+    ti = _field(dims, rng, "2").astype(np.float32)
+    di = np.full(int(np.prod(sdims)), np.nan, np.float32)
+    out = []
+    try:
+        for flow in (1, 0):
+            g2s_amd.set_default_tuning("loop.flow", flow)
+            out.append(g2s_amd.qs(ti, dims, di, sdims, [1], n, 1.2, 3, tie_quantum=2.0 ** (default - finer),
+                                  stage_timing=True))
+    finally:
+        g2s_amd.set_default_tuning("loop.flow", 1)
+    assert out[0][0].tobytes() == out[1][0].tobytes() and out[0][1].tobytes() == out[1][1].tobytes()
+    assert (out[0][2]["gather_ms"] > 0.0) == (finer > 0)
+
+
 @pytest.mark.parametrize("kinds", [("cont",), ("3",), ("cont", "3")])
 def test_flow_gives_up(kinds):
     """A wait that hits its bound (here the first poll that finds a value
