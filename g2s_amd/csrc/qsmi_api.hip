@@ -762,20 +762,33 @@ int qsmi_synchronize(qsmi_device* dev) {
 
 }  // extern "C"
 
+// The direct sum grows with positions x terms (0.25 us a million up to two
+// sub-images, whose loads are in flight together, 0.52 above), the transforms
+// with the sub-images and hardly with the terms. The line lies where the map
+// alone is not slower than by transforms (the search after it gains 40 to 130
+// us besides). Candidate, us, direct / transforms, on both sides of it:
+//   direct:     1000 x 1000, 2 sub-images, 190 neighbours 119 / 110; 4 and 40: 87 / 124; 6 and 40: 130 / 149;
+//               2000 x 2000, 2 and 40: 105 / 167; 180 x 150 x 120, 2 and 40: 84 / 121; 16 and 10: 232 / 288
+//   transforms: 1000 x 1000, 4 and 90: 168 / 131; 6 and 90: 272 / 163; 1400 x 1400, 6 and 40: 272 / 165;
+//               2000 x 2000, 2 and 90: 193 / 182; 180 x 150 x 120, 2 and 90: 162 / 146; 4 and 40: 198 / 146
+static bool node_direct_faster(long long positions, int nb, int V) {
+  const double m = 1e-6 * (double)positions, terms = m * nb * V;
+  const double direct = 17.0 + (V <= 2 ? 0.25 : 0.52) * terms + 2.5 * m;
+  const double transforms = 70.0 + 8.0 * V + (8.0 + 3.5 * V) * m + 0.1 * nb;
+  return direct <= 1.1 * transforms;
+}
+
 // Whether the node's map is summed directly (qsmi_node.hip), with its buffers
 // in place: the exact selection applies (no tie quantum, one finite error
 // bound), positions do not wrap, one layer, and the arguments hold the
 // neighbours. Without memory for the FP64 map the transforms make the map.
-// The direct sum grows with positions x terms, the transforms hardly with the
-// terms: candidate and search together take 218 us against 301 at 648 M terms
-// (180 x 150 x 120, 100 neighbours), 212 against 299 at 360 M in six
-// sub-images, but 1059 against 636 at 3.4 G (3000 x 3000, 190 neighbours).
-constexpr long long kNodeTerms = 1ll << 29;
+// The buffers come with the first such node: a device that scans waves only
+// never needs 8 bytes a position more.
 static bool node_direct(qsmi_device* dev, const NodeInfo& ni) {
   const qsmi_ti* t = dev->ti;
   if (dev->circular || dev->xLayer || !exact_selection_on(dev) || !(ni.eps > 0.f) || !std::isfinite(ni.eps)) return false;
   if ((long long)ni.nb * (t->D + (int)dev->active.size()) > kNodeWords || t->S >= (1ll << 28)) return false;
-  if (t->S * ni.nb * (long long)dev->active.size() > kNodeTerms) return false;
+  if (!node_direct_faster(t->S, ni.nb, (int)dev->active.size())) return false;
   if (!dev->dMapD) {
     if (hipMalloc(&dev->dMapD, (size_t)t->S * sizeof(double)) != hipSuccess ||
         hipMalloc(&dev->dPart, (size_t)kNodeChunks * kMaxK * sizeof(Cand64)) != hipSuccess ||

@@ -166,7 +166,7 @@ int qsmi_candidate_for_pattern(qsmi_device* dev, int nNeighbors, const int* offs
  * error: rms over the FFT grid of TI sub-image a, v_ja the neighbours'
  * alpha-combined values) is rescored in FP64 and the extendK best of those
  * values are returned (as floats); where the map was summed directly in FP64
- * (not circular, no cross layer, at most 2^29 terms) its values are ranked as
+ * (not circular, no cross layer, where that is the faster) its values are ranked as
  * they are, the same result. After a finite value was set with
  * qsmi_set_value_in_error_array(_with_radius) the FP32 map is used as is. */
 int qsmi_search_k_biggest(qsmi_device* dev, float* errors, unsigned* encodedPosition, unsigned extendK, float seed);

@@ -5,6 +5,8 @@ same positions and values. Sizes around a wavefront's and a block's run, both
 widths of the kernel (below and above 2^19 positions), 1-3 dimensions, one,
 two and more sub-images, crowded ties, exclusions, and the two forms of the
 selection on one map."""
+import time
+
 import numpy as np
 import pytest
 
@@ -101,5 +103,42 @@ def test_node_direct(case):
     assert dev.candidate_for_pattern(off, np.ones((2, nsub), np.float32), 0.0)
     assert not np.isfinite(dev.error_map()).any()
     assert np.all(dev.search_k_biggest(K, 0.5)[1] == 0xFFFFFFFF)
+    dev.close()
+    image.close()
+
+
+@pytest.mark.parametrize("dims,nvar,n", [((1000, 1000), 1, 80), ((1000, 1000), 3, 80), ((1400, 1400), 2, 50),
+                                         ((1400, 1400), 3, 40)])
+def test_node_route(dims, nvar, n):
+    """The map by the route that is chosen against the map by transforms (which
+    a tie quantum keeps): within the stated bound of the FP32 map error, and in
+    no more than 1.3 times its time (the rule allows 1.1 in its own model; the
+    least of some passes, so that the rest is room for the timer)."""
+    rng = np.random.default_rng(60 + nvar)
+    ti = rng.standard_normal((int(np.prod(dims)), nvar)).astype(np.float32)
+    types = [0] * nvar
+    sub = g2s_amd.ti_subimages(ti, dims, types)
+    image = g2s_amd.TrainingImage(sub, dims)
+    dev = g2s_amd.AcceleratorDevice(image, g2s_amd.coef_matrix(types)[0])
+    off = np.stack([rng.integers(-12, 13, n) for _ in dims], 1).astype(np.int32)
+    x = rng.standard_normal((n, nvar)).astype(np.float32)
+    vals = np.stack([np.ones_like(x), x], 2).reshape(n, 2 * nvar)
+    us, maps = [], []
+    for quantum in (0.0, 1e-3):
+        dev.set_tie_quantum(quantum)
+        best = np.inf
+        for _ in range(8):
+            t = time.perf_counter()
+            dev.candidate_for_pattern(off, vals, 0.0)
+            best = min(best, time.perf_counter() - t)
+        us.append(best * 1e6)
+        maps.append(dev.error_map().astype(np.float64))
+    print(f"node map {dims} {nvar} variables, {n} neighbours: chosen {us[0]:.0f} us, transforms {us[1]:.0f} us", flush=True)
+    fin = np.isfinite(maps[1])
+    assert np.array_equal(fin, np.isfinite(maps[0]))
+    rms = np.sqrt((sub.reshape(2 * nvar, -1).astype(np.float64) ** 2).mean(1))
+    bound = 4e-5 * float((rms * 2.0 * np.abs(vals).sum(0).max()).sum())
+    assert np.abs(maps[0][fin] - maps[1][fin]).max() <= bound
+    assert us[0] <= 1.3 * us[1]
     dev.close()
     image.close()
