@@ -82,7 +82,7 @@ def test_node_direct(case):
         bound = np.zeros(shape)
         # one rounding to FP32, and FP32 combinations of nsub terms a value
         bound[box] = np.abs(acc) * 2.0 ** -24 + size * (nsub * 2.0 ** -23 if nsub > 2 else 2.0 ** -40)
-        assert np.all(np.abs(got - want)[fin] <= bound[fin] + 1e-30)
+        assert np.all(np.abs(got[fin] - want[fin]) <= bound[fin] + 1e-30)
         e, i = dev.search_k_biggest(K, seed)
         e2, i2 = dev.search_k_biggest_noalloc(K, seed)
         assert np.array_equal(i, i2) and np.array_equal(e, e2)
