@@ -18,7 +18,9 @@ The first two concern scans by transforms, which the data-flow loop does not
 run: their probes take the wave loop (``loop.flow`` 0).
 
 Choices are cached in a JSON file keyed by the geometry; a later call with
-the same cache reads the choice instead of measuring again. The choice is
+the same cache reads the choice instead of measuring again, but for one of
+captured graphs that was not measured against the data-flow loop (a file from
+before that loop), which would switch it off. The choice is
 applied as the process-wide default for the TIs created afterwards.
 ``fft.radix_max`` / ``fft.lognv_max`` change the FP32 rounding of the maps:
 with a continuous variable the exact selection makes the realisation
@@ -36,6 +38,8 @@ from . import TrainingImage, qs, set_default_tuning
 
 DEFAULTS = {"scan.grid1024_min": 320, "fft.radix_max": 13, "fft.lognv_max": 6, "pencil.npb": 1, "loop.graph": 0}
 OWN_GRID_CANDIDATES = (("fft.radix_max", (13, 8, 5)), ("fft.lognv_max", (6, 4, 3)), ("pencil.npb", (1, 2, 4)))
+# cache entry beside the geometries: those whose loop.graph was measured against the data-flow loop
+AGAINST_FLOW = "loop.graph against loop.flow"
 
 
 def geometry_key(ti_dims, var_types, n):
@@ -53,6 +57,14 @@ def load_cache(path):
     if not isinstance(data, dict):
         raise ValueError(f"autotune cache {path}: not a JSON object")
     return data
+
+
+def cached_choice(data, key):
+    """The settings that the cache holds for `key`, or None: measure."""
+    settings = data.get(key)
+    if settings is None or (int(settings.get("loop.graph", 0)) and key not in data.get(AGAINST_FLOW, ())):
+        return None
+    return {k: int(v) for k, v in settings.items()}
 
 
 def save_cache(path, cache):
@@ -106,9 +118,8 @@ def autotune(ti, ti_dims, var_types, n, k, cache=None, sim_dims=None, repeats=3,
     measured) where measured is {description: path loop ms} (empty when the
     choice came from the cache)."""
     key = geometry_key(ti_dims, var_types, n)
-    data = load_cache(cache)
-    if key in data:
-        settings = {k_: int(v) for k_, v in data[key].items()}
+    settings = cached_choice(load_cache(cache), key)
+    if settings is not None:
         apply(settings)
         return settings, {}
     if sim_dims is None:  # a short probe: a few thousand path nodes on the full TI
@@ -139,5 +150,6 @@ def autotune(ti, ti_dims, var_types, n, k, cache=None, sim_dims=None, repeats=3,
     if cache:
         data = load_cache(cache)
         data[key] = best
+        data[AGAINST_FLOW] = sorted({*data.get(AGAINST_FLOW, ()), key})
         save_cache(cache, data)
     return best, measured

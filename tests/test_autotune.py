@@ -21,6 +21,17 @@ def test_cache_roundtrip(tmp_path):
         assert json.load(fh) == data
 
 
+def test_graphs_not_measured_against_the_data_flow_loop_are_measured_again():
+    key, other = "D2:1000x1000:t0:n80", "D2:500x500:t0:n60"
+    waves = dict(autotune.DEFAULTS)
+    graphs = dict(waves, **{"loop.graph": 1})
+    assert autotune.cached_choice({}, key) is None
+    assert autotune.cached_choice({key: waves}, key) == waves
+    assert autotune.cached_choice({key: graphs}, key) is None
+    assert autotune.cached_choice({key: graphs, autotune.AGAINST_FLOW: [other]}, key) is None
+    assert autotune.cached_choice({key: graphs, autotune.AGAINST_FLOW: [key]}, key) == graphs
+
+
 def test_defaults_cover_every_candidate_key():
     keys = {k for k, _ in autotune.OWN_GRID_CANDIDATES} | {"scan.grid1024_min", "loop.graph"}
     assert keys == set(autotune.DEFAULTS)
