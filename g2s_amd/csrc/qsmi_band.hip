@@ -62,10 +62,13 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 // Rescoring tiles of a full-fallback node (slices of its valid box), one
 // wavefront each: a node's box is a serial chain of box / tiles / 64 rounds,
 // so the tail of a wave with one such node is set by their number. 128 -> 1024
-// tiles: 234 -> 67 us a launch of the calibration (1000 x 1000).
-// The per-GPU scratch array of the allocation-free search holds 128.
+// tiles: 234 -> 67 us a launch of the calibration (1000 x 1000). Buffers for
+// more than kFullNodes nodes (whose other nodes fill the chip, and whose tile
+// results would take up to 262 KB each) and the per-GPU scratch array of the
+// allocation-free search hold 128.
 constexpr int kFullTiles = 1024;
-constexpr int kFullTilesScratch = 128;
+constexpr int kFullTilesMany = 128;
+constexpr size_t kFullNodes = 2048;
 constexpr int kSegNodes = 2048;  // nodes per rescoring launch (their tile prefix sums are held in LDS)
 
 // Device view of the band buffers.
@@ -518,6 +521,7 @@ int band_grow(BandBufs* b, int nNodes, int blocksPerNode, int K) {
   const size_t nn = std::max(n, b->capNodes);
   const size_t qq = std::max(q, b->capQueue);
   const int kk = std::max(K, b->K);
+  const int tiles = nn <= kFullNodes ? kFullTiles : kFullTilesMany;
   // grown between launches of one stream: work queued on the old buffers
   // finishes first (the callers' streams do not synchronise with the null
   // stream, so wait for the device before the statistics are read back)
@@ -532,14 +536,14 @@ int band_grow(BandBufs* b, int nNodes, int blocksPerNode, int K) {
       hipMalloc(&b->cnt, nn * sizeof(int)) != hipSuccess || hipMalloc(&b->theta, nn * sizeof(float)) != hipSuccess ||
       hipMalloc(&b->queue, qq * sizeof(int2)) != hipSuccess || hipMalloc(&b->qcnt, 2 * sizeof(int)) != hipSuccess ||
       hipMalloc(&b->val, nn * kBandCap * sizeof(double)) != hipSuccess ||
-      hipMalloc(&b->part, nn * kFullTiles * (size_t)kk * sizeof(Cand64)) != hipSuccess ||
+      hipMalloc(&b->part, nn * tiles * (size_t)kk * sizeof(Cand64)) != hipSuccess ||
       hipMalloc(&b->stats, sizeof(keep)) != hipSuccess ||
       hipMemcpy(b->stats, keep, sizeof(keep), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(b->qcnt, zero, sizeof(zero), hipMemcpyHostToDevice) != hipSuccess) {
     band_free(b);
     return fail(QSMI_ERR_NOMEM, "exact selection buffers: out of device memory");
   }
-  b->tiles = kFullTiles;
+  b->tiles = tiles;
   b->capNodes = nn;
   b->capQueue = qq;
   b->K = kk;
@@ -552,7 +556,7 @@ int band_grow(BandBufs* b, int nNodes, int blocksPerNode, int K) {
 size_t band_scratch_bytes(int K) {
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   return al(kBandCap * sizeof(uint32_t)) + 2 * al(sizeof(int)) + al(sizeof(float)) + al(sizeof(int2)) +
-         al(kBandCap * sizeof(double)) + al((size_t)kFullTilesScratch * K * sizeof(Cand64)) +
+         al(kBandCap * sizeof(double)) + al((size_t)kFullTilesMany * K * sizeof(Cand64)) +
          al(4 * sizeof(unsigned long long));
 }
 
@@ -572,9 +576,9 @@ void band_view(BandBufs* b, void* base, int K) {
   b->val = reinterpret_cast<double*>(p);
   p += al(kBandCap * sizeof(double));
   b->part = reinterpret_cast<Cand64*>(p);
-  p += al((size_t)kFullTilesScratch * K * sizeof(Cand64));
+  p += al((size_t)kFullTilesMany * K * sizeof(Cand64));
   b->stats = reinterpret_cast<unsigned long long*>(p);
-  b->tiles = kFullTilesScratch;
+  b->tiles = kFullTilesMany;
   b->capNodes = 1;
   b->capQueue = 1;
   b->K = K;

@@ -470,3 +470,31 @@ def test_cross_layer_per_node(dims, nv, nb):
         ov, op, _ = oracle.select_device(dims, M.astype(np.float32), lo, hi, K, 0.37)
         assert np.array_equal(pos, op.astype(np.int64)) and np.array_equal(err, ov)
     dev.close()
+
+
+def test_wave_of_many_nodes_full_rescoring():
+    """A wave of 4096 nodes, 16 best, on an image whose 10,000 positions all
+    tie (every list overflows and the whole box is rescored): the selection is
+    that of the same nodes in a small wave (which cuts the box into more
+    tiles), and the buffers stay at 98 + 32 KB a node (lists, tile results)
+    and the scan's own."""
+    import torch
+
+    rng = np.random.default_rng(77)
+    dims, K, n = (100, 100), 16, 4096
+    ti = np.full(dims[0] * dims[1], 0.75, np.float32)
+    image = g2s_amd.TrainingImage(g2s_amd.ti_subimages(ti, dims, [0]), dims)
+    dev = g2s_amd.AcceleratorDevice(image, g2s_amd.coef_matrix([0])[0])
+    off = np.array([[0, 0], [1, -1]], np.int32)
+    vals = np.array([[1.0, 0.5], [1.0, 0.25]], np.float32)
+    nodes = [(off, vals, -0.3125, float(s)) for s in rng.random(n, np.float32)]
+    small = [np.asarray(a) for a in dev.scan_wave(nodes[:64], K)]
+    free = torch.cuda.mem_get_info()[0]
+    e, p, c = dev.scan_wave(nodes, K)
+    used = free - torch.cuda.mem_get_info()[0]
+    _log(f"4096 nodes, 16 best: {used / n / 1024:.0f} KB a node more on the device")
+    assert np.array_equal(e[:64], small[0]) and np.array_equal(p[:64], small[1]) and np.array_equal(c[:64], small[2])
+    scan = 2 * (dims[0] // 2 + 1) * dims[1] * 8  # two half spectra of the scan
+    assert used < n * (130 * 1024 + scan + 64 * 1024)
+    dev.close()
+    image.close()
