@@ -10,6 +10,7 @@ Selection with a tie quantum (categorical TIs) stays in FP32: bit-exact
 against the device rule on the same GPU map, and against the FP64 map equal
 except where the two FP64 values are within quantum + 2 eps.
 """
+import ctypes
 import sys
 
 import numpy as np
@@ -478,7 +479,10 @@ def test_wave_of_many_nodes_full_rescoring():
     that of the same nodes in a small wave (which cuts the box into more
     tiles), and the buffers stay at 98 + 32 KB a node (lists, tile results)
     and the scan's own."""
-    import torch
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert g2s_amd.lib().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0  # the library's HIP runtime
+        return free.value
 
     rng = np.random.default_rng(77)
     dims, K, n = (100, 100), 16, 4096
@@ -489,9 +493,9 @@ def test_wave_of_many_nodes_full_rescoring():
     vals = np.array([[1.0, 0.5], [1.0, 0.25]], np.float32)
     nodes = [(off, vals, -0.3125, float(s)) for s in rng.random(n, np.float32)]
     small = [np.asarray(a) for a in dev.scan_wave(nodes[:64], K)]
-    free = torch.cuda.mem_get_info()[0]
+    free = free_bytes()
     e, p, c = dev.scan_wave(nodes, K)
-    used = free - torch.cuda.mem_get_info()[0]
+    used = free - free_bytes()
     _log(f"4096 nodes, 16 best: {used / n / 1024:.0f} KB a node more on the device")
     assert np.array_equal(e[:64], small[0]) and np.array_equal(p[:64], small[1]) and np.array_equal(c[:64], small[2])
     scan = 2 * (dims[0] // 2 + 1) * dims[1] * 8  # two half spectra of the scan
