@@ -64,6 +64,12 @@ CASES = [
     (("3",), (40, 33, 12), (10, 9, 7), 40, 1.5, dict(kimg=True)),
     (("3",), (400,), (90,), 11, 1.5, {}),
     (("2", "3"), (60, 45), (15, 14), 20, 16.0, dict(partial=True, quantum=0.0)),
+    # three and four variables, continuous ones among them
+    (("cont", "3", "cont"), (52, 47), (14, 12), 15, 3.0, dict(partial=True, hard=0.05)),
+    (("cont", "2", "cont", "3"), (40, 38), (12, 11), 9, 9.0, dict(weights="distance")),
+    # several slices a node: counts, mixed
+    (("2",), (250, 250), (40, 40), 50, 1.2, {}),
+    (("cont", "4"), (200, 190), (24, 20), 40, 1.5, dict(hard=0.1)),
 ]
 
 
@@ -121,6 +127,23 @@ def test_flow_then_waves(case):
         g2s_amd.set_default_tuning("loop.flow", 1)
     assert a[0].tobytes() == b[0].tobytes() and a[1].tobytes() == b[1].tobytes()
     assert a[2]["gather_ms"] > 0.0 and a[2]["waves"] == b[2]["waves"]
+
+
+@pytest.mark.parametrize("kind", ["cont", "3"])
+def test_flow_without_valid_position(kind):
+    """Kernels larger than the image: many nodes have no position whose
+    neighbours all lie inside it; their cells stay empty and give their
+    neighbours nothing."""
+    rng = np.random.default_rng(17)
+    dims, sdims, kd = (9, 7), (25, 20), [21, 21]
+    ti = _field(dims, rng, kind).astype(np.float32)
+    di = np.full(int(np.prod(sdims)), np.nan, np.float32)
+    kw = dict(kernel=np.ones(kd[0] * kd[1], np.float32), kernel_dims=kd)
+    args = (ti, dims, di, sdims, [0 if kind == "cont" else 1], 6, 2.0, 3)
+    _both(*args, **kw)
+    empty = int(np.isnan(g2s_amd.qs(*args, **kw)[0]).sum())
+    print(f"data-flow loop: {empty} of {di.size} cells without a valid position", flush=True)
+    assert 0 < empty < di.size
 
 
 def test_flow_slices_and_segments():
