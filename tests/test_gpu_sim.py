@@ -31,6 +31,19 @@ def _log(m):
     sys.stdout.flush()
 
 
+@pytest.fixture(params=["flow", "waves"])
+def loop(request):
+    """Both path loops, where a request qualifies for the data-flow loop."""
+    g2s_amd.set_default_tuning("loop.flow", int(request.param == "flow"))
+    yield request.param
+    g2s_amd.set_default_tuning("loop.flow", 1)
+
+
+def ran(st):
+    """Which loop a run with stage timing took: only waves have a gather stage."""
+    return "waves" if st["gather_ms"] > 0.0 else "flow"
+
+
 def default_kernel(ti_dims, nexp):
     kd = [d // 2 + 1 for d in ti_dims]
     return kd, np.ones(int(np.prod(kd)) * nexp, np.float32)
@@ -38,8 +51,9 @@ def default_kernel(ti_dims, nexp):
 
 def lockstep(ti, ti_dims, di0, sim_dims, types, n, k, seed, quantum, nodes=None,
              weights=None, wave_size=64, threads=8, cross=False, no_verbatim=False, n_image=None, k_image=None,
-             circular_sim=False, circular_ti=False):
-    """nodes: path-relative node indices to check (None: every node);
+             circular_sim=False, circular_ti=False, loop=None):
+    """loop: the path loop that the run is expected to take (None: any);
+    nodes: path-relative node indices to check (None: every node);
     weights: one kernel weight per variable (None: the default uniform 1)."""
     types = list(types)
     nvar = len(types)
@@ -49,8 +63,9 @@ def lockstep(ti, ti_dims, di0, sim_dims, types, n, k, seed, quantum, nodes=None,
         gkw = dict(kernel=np.tile(np.asarray(weights, np.float32), int(np.prod(kd0))), kernel_dims=kd0)
     sim, idx, st = g2s_amd.qs(ti, ti_dims, di0, sim_dims, types, n, k, seed, wave_size=wave_size,
                               tie_quantum=quantum, no_verbatim=no_verbatim, n_image=n_image, k_image=k_image,
-                              circular_sim=circular_sim, circular_ti=circular_ti, **gkw)
+                              circular_sim=circular_sim, circular_ti=circular_ti, stage_timing=loop is not None, **gkw)
     _log(f"  gpu run: {st}")
+    assert loop is None or ran(st) == loop
     # oracle set-up identical to the reference's qs.cpp
     ncat, catvals = [], []
     for v in range(nvar):
@@ -190,26 +205,26 @@ def test_sim_no_verbatim(kind):
     assert hp > 0
 
 
-def test_sim_continuous_2d():
+def test_sim_continuous_2d(loop):
     g = synth.grf((48, 56), 4.0, seed=21)
     ti, dims = synth.to_g2s(np.exp(g))
     sdims = (40, 36)
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     _log("continuous 2-D")
-    lockstep(ti, dims, di, sdims, [0], 20, 1.5, 7, 0.0)
+    lockstep(ti, dims, di, sdims, [0], 20, 1.5, 7, 0.0, loop=loop)
 
 
-def test_sim_categorical_2d():
+def test_sim_categorical_2d(loop):
     g = synth.grf((50, 50), 5.0, seed=22, anis=(3.0,), angle_deg=30.0)
     ti, dims = synth.to_g2s((g > np.quantile(g, 0.72)).astype(np.float32))
     sdims = (40, 40)
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     q = float(2.0 ** (np.ceil(np.log2(15)) - 16))
     _log("categorical 2-D")
-    lockstep(ti, dims, di, sdims, [1], 15, 1.2, 3, q)
+    lockstep(ti, dims, di, sdims, [1], 15, 1.2, 3, q, loop=loop)
 
 
-def test_sim_multivariate_hard_data():
+def test_sim_multivariate_hard_data(loop):
     a = synth.grf((40, 44), 4.0, seed=23)
     b_ = synth.grf((40, 44), 4.0, seed=24)
     c = 0.7 * a + 0.71 * b_
@@ -221,10 +236,10 @@ def test_sim_multivariate_hard_data():
     pick = rng.choice(di.shape[0], size=di.shape[0] // 10, replace=False)
     di[pick] = ti[rng.integers(0, ti.shape[0], size=pick.size)]
     _log("multivariate 2-D with hard data")
-    lockstep(ti, dims, di.reshape(-1), sdims, [0, 1], 12, 1.5, 4, 0.0)
+    lockstep(ti, dims, di.reshape(-1), sdims, [0, 1], 12, 1.5, 4, 0.0, loop=loop)
 
 
-def test_sim_categorical_3d():
+def test_sim_categorical_3d(loop):
     g1 = synth.grf((12, 16, 18), (3.0, 5.0, 5.0), seed=25)
     fac = (g1 > np.quantile(g1, 0.5)).astype(np.float32) + (g1 > np.quantile(g1, 0.8)).astype(np.float32)
     ti, dims = synth.to_g2s(fac)
@@ -232,16 +247,16 @@ def test_sim_categorical_3d():
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     q = float(2.0 ** (np.ceil(np.log2(20)) - 16))
     _log("categorical 3-D")
-    lockstep(ti, dims, di, sdims, [1], 20, 1.5, 9, q)
+    lockstep(ti, dims, di, sdims, [1], 20, 1.5, 9, q, loop=loop)
 
 
-def test_sim_1d():
+def test_sim_1d(loop):
     g = synth.grf((300,), 6.0, seed=26)
     ti, dims = synth.to_g2s(np.exp(g))
     sdims = (200,)
     di = np.full(200, np.nan, np.float32)
     _log("continuous 1-D")
-    lockstep(ti, dims, di, sdims, [0], 10, 1.5, 11, 0.0)
+    lockstep(ti, dims, di, sdims, [0], 10, 1.5, 11, 0.0, loop=loop)
 
 
 def test_sim_nan_ti_continuous_2d():
@@ -322,7 +337,7 @@ def test_sim_several_tis():
 
 
 @pytest.mark.parametrize("kind", ["continuous", "categorical"])
-def test_sim_n_and_k_images(kind):
+def test_sim_n_and_k_images(kind, loop):
     """qs -ni / -kvi: per-cell n and k, lockstep with the oracle's serial loop."""
     if kind == "continuous":
         g = synth.grf((48, 56), 4.0, seed=51)
@@ -339,10 +354,10 @@ def test_sim_n_and_k_images(kind):
     kimg = rng.choice([1.0, 2.0, 3.5, 0.0], cells).astype(np.float32)
     di = np.full(cells, np.nan, np.float32)
     _log(f"n / k images {kind}: n in (4, 9, 20), k in (1, 2, 3.5, run's 1.5)")
-    lockstep(ti, dims, di, sdims, types, 20, 1.5, 8, q, n_image=nimg, k_image=kimg)
+    lockstep(ti, dims, di, sdims, types, 20, 1.5, 8, q, n_image=nimg, k_image=kimg, loop=loop)
 
 
-def test_sim_kernel_index_image():
+def test_sim_kernel_index_image(loop):
     """qs -ki a b -kii image: each cell's kernel (weights and its own offset
     order); lockstep with the oracle node by node (one oracle per kernel,
     the node's kernel deciding), and an index image of zeros gives the
@@ -364,7 +379,8 @@ def test_sim_kernel_index_image():
     n, k, seed = 16, 1.5, 12
     _log("kernel-index image: 21x21 uniform / 15x11 exponential, random per cell")
     sim, idx, st = g2s_amd.qs(ti, dims, di, sdims, [0], n, k, seed, wave_size=64, kernels=[k0, k1], kernels_dims=kd,
-                              kernel_index_image=kii)
+                              kernel_index_image=kii, stage_timing=True)
+    assert ran(st) == loop
     informed = (~np.isnan(di)).astype(np.uint8)
     p, s_, b = oracle.path(informed, seed)
     sims = [oracle.Sim(ti, dims, [0], [], [], sdims, kdq, kq, oracle.offsets(kdq, kq), n, k, p, s_, b)
@@ -387,7 +403,7 @@ def test_sim_kernel_index_image():
 
 
 @pytest.mark.parametrize("kind", ["continuous", "categorical_no_verbatim"])
-def test_sim_circular_simulation(kind):
+def test_sim_circular_simulation(kind, loop):
     """qs -csim: neighbours wrap around the simulation grid; lockstep with
     the oracle's serial loop (with -nV on top in the categorical case)."""
     if kind == "continuous":
@@ -401,7 +417,8 @@ def test_sim_circular_simulation(kind):
     sdims = (40, 36)
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     _log(f"circular simulation {kind}")
-    lockstep(ti, dims, di, sdims, types, 15, 1.5, 9, q, circular_sim=True, no_verbatim=nv)
+    lockstep(ti, dims, di, sdims, types, 15, 1.5, 9, q, circular_sim=True, no_verbatim=nv,
+             loop="waves" if nv else loop)
 
 
 @pytest.mark.parametrize("kind", ["continuous", "categorical"])
@@ -498,7 +515,7 @@ def test_sim_several_tis_of_their_own_extents():
 
 
 @pytest.mark.parametrize("kind", ["continuous_1000", "categorical_generic"])
-def test_sim_bit_reproducible(kind):
+def test_sim_bit_reproducible(kind, loop):
     """One seeded realisation run twice gives identical bytes (simulation and
     index image): every FP32 sum of the scan has a fixed order, and the exact
     selection depends on FP64 values only."""
@@ -513,17 +530,19 @@ def test_sim_bit_reproducible(kind):
         sdims = (40, 40)
     di = np.full(int(np.prod(sdims)), np.nan, np.float32)
     _log(f"bit reproducibility {kind}: two runs of seed 3")
-    s1, i1, _ = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 3, wave_size=256, tie_quantum=q)
+    s1, i1, st = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 3, wave_size=256, tie_quantum=q, stage_timing=True)
+    assert ran(st) == loop
     s2, i2, _ = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 3, wave_size=256, tie_quantum=q)
     assert s1.tobytes() == s2.tobytes() and i1.tobytes() == i2.tobytes()
 
 
 @pytest.mark.parametrize("kind", ["continuous_1000", "categorical_generic"])
-def test_sim_wave_size_invariant(kind):
+def test_sim_wave_size_invariant(kind, loop):
     """The realisation does not depend on how path nodes are packed into
     waves: 16-node waves (several waves per dependency level, alternating
     between the loop's two streams), 256-node waves, and one wave per level
-    (one stream) give identical bytes."""
+    (one stream) give identical bytes. In the data-flow loop the size bounds the
+    nodes in flight and the nodes of a launch."""
     if kind == "continuous_1000":
         w = synth.config2_continuous_2d()
         ti, dims, types, n, k, q = w["ti"], w["ti_dims"], [0], 80, 1.5, 0.0
@@ -537,7 +556,9 @@ def test_sim_wave_size_invariant(kind):
     runs = []
     for ws in (16, 256, 1 << 20):
         _log(f"wave-size invariance {kind}: waves of <= {ws} nodes")
-        s, i, st = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 5, wave_size=ws, tie_quantum=q)
+        s, i, st = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 5, wave_size=ws, tie_quantum=q,
+                               stage_timing=True)
+        assert ran(st) == loop
         runs.append((s.tobytes(), i.tobytes(), st["waves"]))
     assert runs[0][2] > runs[2][2] and runs[1][2] >= runs[2][2]
     for s, i, _ in runs[1:]:
@@ -561,18 +582,22 @@ def test_sim_graph_steps_identical(kind):
         sdims, di = c["sim_dims"], c["di"]
         kd0 = [d // 2 + 1 for d in dims]  # weights 0.5 / 0.5
         gkw = dict(kernel=np.tile(np.asarray([0.5, 0.5], np.float32), int(np.prod(kd0))), kernel_dims=kd0)
+    g2s_amd.set_default_tuning("loop.flow", 0)  # launched waves beside the captured ones
     try:
         for ws in (16, 256):
             runs = []
             for graph in (0, 1):
                 g2s_amd.set_default_tuning("loop.graph", graph)
                 _log(f"graph steps {kind}: waves of <= {ws} nodes, loop.graph={graph}")
-                s, i, st = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 9, wave_size=ws, **gkw)
+                s, i, st = g2s_amd.qs(ti, dims, di, sdims, types, n, k, 9, wave_size=ws,
+                                       stage_timing=not graph, **gkw)
+                assert graph or ran(st) == "waves"
                 runs.append((s.tobytes(), i.tobytes(), st["waves"]))
             assert runs[0][2] == runs[1][2] and runs[0][2] > 1
             assert runs[1][0] == runs[0][0] and runs[1][1] == runs[0][1]
     finally:
         g2s_amd.set_default_tuning("loop.graph", 0)
+        g2s_amd.set_default_tuning("loop.flow", 1)
 
 
 def _partial_grid(sdims, nvar, rng, frac_partial=0.3, frac_full=0.05, src=None):
@@ -596,7 +621,7 @@ def _partial_grid(sdims, nvar, rng, frac_partial=0.3, frac_full=0.05, src=None):
 
 
 @pytest.mark.parametrize("kind", ["multivariate_generic", "continuous_1024", "centre_only"])
-def test_sim_partially_informed_cells(kind):
+def test_sim_partially_informed_cells(kind, loop):
     """Partially informed simulation cells (include/simulation.hpp:324-335,
     581-584, 658-666): simulated at their place in the path with their own
     values as the centre neighbour, keeping them. Lockstep against the
@@ -625,7 +650,7 @@ def test_sim_partially_informed_cells(kind):
     _log(f"partially informed cells {kind}: TI {dims}, sim {sdims}, n={n}")
     free = int(np.isnan(di.reshape(-1, nvar)).any(axis=1).sum())  # the path nodes
     nodes = None if kind != "continuous_1024" else _sample_nodes(free, 400, 5)
-    lockstep(ti, dims, di, sdims, types, n, k, 13, 0.0, nodes=nodes, wave_size=64, threads=8)
+    lockstep(ti, dims, di, sdims, types, n, k, 13, 0.0, nodes=nodes, wave_size=64, threads=8, loop=loop)
 
 
 def _sample_nodes(total, count, seed):
