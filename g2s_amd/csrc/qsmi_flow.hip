@@ -1550,7 +1550,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   }
   size_t countFrom = judge ? 0 : nPath, verdict = (size_t)std::max(64, R.n);  // nodes counted, then judged
   unsigned long long seen[kFlowStats] = {};
-  size_t done = 0;
+  size_t done = 0, judgedAt = 0;
   const size_t stop = t->tune.flowNodes > 0 ? std::min(nPath, (size_t)t->tune.flowNodes) : nPath;
   for (size_t b = 0; b < stop && e == hipSuccess && !slow; b = done) {
     P.node0 = (int)b;
@@ -1590,12 +1590,23 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
       e = hipStreamSynchronize(st);
       if (e == hipSuccess) e = hipMemcpy(sv, P.stats, sizeof(sv), hipMemcpyDeviceToHost);
       if (e != hipSuccess) break;
-      const double nodes = (double)(done - countFrom), tiles = (double)(sv[4] - seen[4]) / nodes, full = (double)(sv[6] - seen[6]) / nodes;
+      const double nodes = (double)(done - countFrom);
+      const double tiles = (double)(sv[4] - seen[4]) / nodes, full = (double)(sv[6] - seen[6]) / nodes;
       double steps = (double)(sv[5] - seen[5]) / nodes;
       // the first lists are short: what comes after the first step grows with them
-      if (countFrom == 0 && full > tiles) steps = tiles + (steps - tiles) * std::max(1.0, tiles * (maxSteps - 1.0) / (full - tiles));
-      slow = flow_path_us(F, R, done, flow_cost(tiles, steps, terms, R.nVar, P.K, P.G)) >
-             kHandOver * wave_path_us(F, R, done);
+      if (countFrom == 0 && full > tiles)
+        steps = tiles + (steps - tiles) * std::max(1.0, tiles * (maxSteps - 1.0) / (full - tiles));
+      // An image of ties (zeros, plateaus) fills the scan's lists before their
+      // end. The wave loop's lists overflow there too and it rescores whole
+      // boxes, some 200 us a node, which its cost does not hold: no hand-over
+      // where a node flushes more than one list. 1000 x 1000, 80 neighbours,
+      // correlation length 20, us a node, direct / waves: 40 % zeros 11 / 41 (10
+      // best 35 / 102), 70 % 12 / 44 (67 / 86), 95 % 46 / 155 (258 / 227); they
+      // flush 10 to 3000 lists, noise none.
+      const bool ties = sv[3] - seen[3] > done - judgedAt;
+      const FlowCost cost = flow_cost(tiles, steps, terms, R.nVar, P.K, P.G);
+      slow = !ties && flow_path_us(F, R, done, cost) > kHandOver * wave_path_us(F, R, done);
+      judgedAt = done;
       memcpy(seen, sv, sizeof(sv));
       countFrom = done < 65536 ? done : done + 65536;
       verdict = done < 65536 ? 4 * done : countFrom + 8192;

@@ -225,25 +225,29 @@ def test_flow_gives_up_at_once():
     assert ms["given up"] < 1.5 * ms["waves"]
 
 
-@pytest.mark.parametrize("kinds,n,sdims,over", [
-    (("noise",), 80, (530, 500), True),
-    (("noise",), 250, (120, 120), True),
-    (("noise", "noise"), 60, (100, 100), True),
-    (("cont",), 80, (150, 150), False),
+@pytest.mark.parametrize("kinds,n,k,sdims,over", [
+    (("noise",), 80, 1.5, (530, 500), True),
+    (("noise",), 250, 1.5, (120, 120), True),
+    (("noise", "noise"), 60, 1.5, (100, 100), True),
+    (("noise",), 80, 10.0, (120, 120), True),
+    (("cont",), 80, 1.5, (150, 150), False),
+    (("zeros",), 80, 10.0, (100, 100), False),
 ])
-def test_flow_hands_over_to_waves(kinds, n, sdims, over):
+def test_flow_hands_over_to_waves(kinds, n, k, sdims, over):
     """1000 x 1000 images: white noise, where the wave loop takes over the rest
-    of the path, and a smooth image, where it does not."""
+    of the path, a smooth image and one of mostly zeros (whose ties overflow
+    the wave loop's lists), where it does not."""
     rng = np.random.default_rng(8)
     dims = (1000, 1000)
-    ti = [rng.standard_normal(dims[0] * dims[1]) if q == "noise" else _field(dims, rng, q) for q in kinds]
+    ti = [rng.standard_normal(dims[0] * dims[1]) if q == "noise" else
+          np.maximum(_field(dims, rng, "cont") - 5.0, 0.0) if q == "zeros" else _field(dims, rng, q) for q in kinds]
     ti = np.stack(ti, 1).astype(np.float32)
     di = np.full((sdims[0] * sdims[1], len(kinds)), np.nan, np.float32)
     out = []
     try:
         for flow in (1, 0):
             g2s_amd.set_default_tuning("loop.flow", flow)
-            out.append(g2s_amd.qs(ti, dims, di, sdims, [0] * len(kinds), n, 1.5, 6, stage_timing=True))
+            out.append(g2s_amd.qs(ti, dims, di, sdims, [0] * len(kinds), n, k, 6, stage_timing=True))
     finally:
         g2s_amd.set_default_tuning("loop.flow", 1)
     assert out[0][0].tobytes() == out[1][0].tobytes() and out[0][1].tobytes() == out[1][1].tobytes()
