@@ -61,6 +61,10 @@ constexpr uint32_t kPending = 0xFFFFFFFFu;  // grid word of a variable not simul
 constexpr uint32_t kEmpty = 0x7FC00000u;    // simulated, but no position was valid
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr uint32_t kNoTicket = 0x40000000u;  // above every ticket of a launch (nodes x slices)
+// The word that says so stands in a cache line of its own: waits look at it, and
+// beside the ticket, which every block adds to, that look slowed the tickets
+// (500 x 500, 5 classes and a continuous variable, 60 x 60 nodes: 30 -> 20 ms).
+constexpr int kGaveUp = 64, kCtlWords = 128;
 constexpr unsigned long long kOpen = ~0ull;  // slice result not written yet
 constexpr int kThreads = 256, kWaves = kThreads / 64;
 // A wavefront sums kPair tiles of kTileX x kTileY positions side by side; the
@@ -103,7 +107,7 @@ struct FlowParams {
   const float* di;    // the grid as given
   uint32_t* work;     // the grid under simulation
   uint32_t* index;
-  int* ctl;           // [0] ticket (kNoTicket and above: none left), [1] a wait was given up
+  int* ctl;           // [0] ticket (kNoTicket and above: none left), [kGaveUp] a wait was given up
   int polls;          // polls after which a wait is given up
   unsigned long long* slots;
   unsigned long long* stats;  // [kFlowStats]: nodes, positions scored, 0, flushes; tiles, their steps, without the bound
@@ -134,34 +138,31 @@ __device__ __forceinline__ void st_agent64(unsigned long long* p, unsigned long 
 }
 
 // Bounded wait step: false when the wait is given up. Then every other wait of
-// the kernel ends as well and no block takes another ticket (what the other
-// nodes would be simulated from is not valid). The ticket itself says so: a
-// look at ctl[1] with every ticket, beside the line that all blocks add to,
-// took the loop from 143 to 225 ms (220 x 220 nodes of a 1000 x 1000 image).
-__device__ __forceinline__ bool poll_again(int& polls, int bound, int* ctl) {
+// the kernel ends as well, and the next node that is written ends the tickets
+// (end_tickets): what the other nodes would be simulated from is not valid.
+__device__ __forceinline__ bool poll_again(int& polls, int bound, int* err) {
   if (++polls >= bound) {
-    st_agent((uint32_t*)&ctl[1], 1u);
-    st_agent((uint32_t*)&ctl[0], kNoTicket);
+    st_agent((uint32_t*)err, 1u);
     return false;
   }
-  if ((polls & 63) == 0 && ld_agent((const uint32_t*)&ctl[1])) return false;
+  if ((polls & 63) == 0 && ld_agent((const uint32_t*)err)) return false;
   __builtin_amdgcn_s_sleep(2);
   return true;
 }
 
-__device__ __forceinline__ uint32_t wait_word(const uint32_t* p, int bound, int* ctl) {
+__device__ __forceinline__ uint32_t wait_word(const uint32_t* p, int bound, int* err) {
   uint32_t b = ld_agent(p);
   for (int polls = 0; b == kPending;) {
-    if (!poll_again(polls, bound, ctl)) return kEmpty;
+    if (!poll_again(polls, bound, err)) return kEmpty;
     b = ld_agent(p);
   }
   return b;
 }
 
-__device__ __forceinline__ unsigned long long wait_word64(const unsigned long long* p, int bound, int* ctl) {
+__device__ __forceinline__ unsigned long long wait_word64(const unsigned long long* p, int bound, int* err) {
   unsigned long long b = ld_agent64(p);
   for (int polls = 0; b == kOpen;) {
-    if (!poll_again(polls, bound, ctl)) return kOpen;
+    if (!poll_again(polls, bound, err)) return kOpen;
     b = ld_agent64(p);
   }
   return b;
@@ -214,6 +215,13 @@ __device__ void write_cell(FlowArgs& P, unsigned cell, uint32_t p) {
     if (!isnan(P.di[c + v])) continue;  // a given value is kept
     st_agent(&P.work[c + v], p == kNone ? kEmpty : __float_as_uint(P.tiVals[(long long)p * P.nVar + v]));
   }
+}
+
+// No block takes another ticket once a wait has been given up. Looked at once a
+// node, by the thread that has written it: with every ticket that look cost up
+// to half of the loop's rate.
+__device__ __forceinline__ void end_tickets(FlowArgs& P) {
+  if (ld_agent((const uint32_t*)&P.ctl[kGaveUp])) st_agent((uint32_t*)&P.ctl[0], kNoTicket);
 }
 
 // The rank draw over the K best (best first), as draw_write of qsmi_select.hpp.
@@ -282,7 +290,7 @@ __device__ __forceinline__ void gather_node(FlowArgs& P, int i, unsigned cell, i
       if (v >= P.nVar) continue;
       uint32_t b = bits[v];
       if (b == kPending && t != cell) {
-        b = wait_word(&wp[v], P.polls, P.ctl);
+        b = wait_word(&wp[v], P.polls, &P.ctl[kGaveUp]);
         waited = true;
       }
       val[v] = (b == kPending || b == kEmpty) ? NAN : __uint_as_float(b);
@@ -551,7 +559,7 @@ __device__ __forceinline__ float uniform(float v) {
 // COUNT: tiles and steps are counted (a scalar more in the tile loop, 1 % of the
 // scan, so only the segments that are judged by them do).
 template <int FORM, int NV, int KT, bool COUNT>
-__global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_flow_direct(FlowParams kernArgs) {
+__global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 && FORM != 2 ? 6 : 5) : 4) k_flow_direct(FlowParams kernArgs) {
   constexpr bool MIXED = FORM == 2;
   extern __shared__ __align__(16) char dyn[];
   __shared__ FlowShared sh;
@@ -931,8 +939,8 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
       if (tid < K) tk.push(best[tid]);
       for (int e = tid; e < (G - 1) * K; e += kThreads) {
         Cand64 c;
-        c.pos = (uint32_t)wait_word64(&sl[(long long)e * 2 + 1], P.polls, P.ctl);
-        c.val = __longlong_as_double((long long)wait_word64(&sl[(long long)e * 2], P.polls, P.ctl));
+        c.pos = (uint32_t)wait_word64(&sl[(long long)e * 2 + 1], P.polls, &P.ctl[kGaveUp]);
+        c.val = __longlong_as_double((long long)wait_word64(&sl[(long long)e * 2], P.polls, &P.ctl[kGaveUp]));
         c.h = tie_hash(seedbits, c.pos);
         if (c.pos != kNone) tk.push(c);
       }
@@ -941,7 +949,10 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 ? 6 : 5) : 4) k_f
     }
     if (tid < K) sh.pos[tid] = best[tid].pos;
     __syncthreads();
-    if (tid == 0) write_cell(P, cell, draw_rank(P, i, seed, sh.pos));
+    if (tid == 0) {
+      write_cell(P, cell, draw_rank(P, i, seed, sh.pos));
+      end_tickets(P);
+    }
     ++nNodesDone;
   }
   if (lane == 0 && nScored) atomicAdd(&P0.stats[1], nScored);
@@ -1267,11 +1278,14 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
           }
       };
       if (tid < K) push((bestR[tid] >> 32 << 32) | sh.pos[tid]);
-      for (int e = tid; e < (G - 1) * K; e += kThreads) push(wait_word64(&sl[e], P.polls, P.ctl));
+      for (int e = tid; e < (G - 1) * K; e += kThreads) push(wait_word64(&sl[e], P.polls, &P.ctl[kGaveUp]));
       __syncthreads();  // bestR and sh.pos have been read
       block_best();
     }
-    if (tid == 0) write_cell(P, cell, draw_rank(P, i, seed, sh.pos));
+    if (tid == 0) {
+      write_cell(P, cell, draw_rank(P, i, seed, sh.pos));
+      end_tickets(P);
+    }
   }
 }
 
@@ -1280,7 +1294,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
 // ---------------------------------------------------------------------------
 // the tickets of the next launch; none after a given-up wait
 __global__ void k_flow_next(int* ctl) {
-  if (ctl[1] == 0) ctl[0] = 0;
+  if (ctl[kGaveUp] == 0) ctl[0] = 0;
 }
 
 __global__ void k_flow_grid(const float* __restrict__ di, uint32_t* __restrict__ work, long long n) {
@@ -1488,7 +1502,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
     return p;
   };
   P.work = (uint32_t*)alloc(SD * R.nVar * sizeof(uint32_t));
-  P.ctl = (int*)alloc(2 * sizeof(int));
+  P.ctl = (int*)alloc(kCtlWords * sizeof(int));
   P.stats = (unsigned long long*)alloc(kFlowStats * sizeof(unsigned long long));
   P.slots = (unsigned long long*)alloc(slotWords * sizeof(unsigned long long));
   float* planes = F.count ? nullptr : (float*)alloc((size_t)R.nVar * t->S * sizeof(float));
@@ -1504,7 +1518,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
     e = hipMemcpy(dq, F.quant.data(), F.quant.size() * sizeof(float), hipMemcpyHostToDevice);
     P.quant = dq;
   }
-  if (e == hipSuccess) e = hipMemsetAsync(P.ctl, 0, 2 * sizeof(int), st);
+  if (e == hipSuccess) e = hipMemsetAsync(P.ctl, 0, kCtlWords * sizeof(int), st);
   if (e == hipSuccess) e = hipMemsetAsync(P.stats, 0, kFlowStats * sizeof(unsigned long long), st);
   const long long words = (long long)SD * R.nVar;
   hipLaunchKernelGGL(k_flow_grid, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, R.dDi, P.work, words);
@@ -1625,14 +1639,14 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
     if (x) (void)hipEventDestroy(x);
   hipLaunchKernelGGL(k_flow_finish, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, R.dDi, P.work, words);
   if (e == hipSuccess) e = hipGetLastError();
-  int ctl[2] = {0, 0};
+  int gone = 0;
   unsigned long long sv[kFlowStats] = {};
   const hipError_t es = hipStreamSynchronize(st);
   if (e == hipSuccess) e = es;
-  if (e == hipSuccess) e = hipMemcpy(ctl, P.ctl, sizeof(ctl), hipMemcpyDeviceToHost);
+  if (e == hipSuccess) e = hipMemcpy(&gone, P.ctl + kGaveUp, sizeof(gone), hipMemcpyDeviceToHost);
   if (e == hipSuccess) e = hipMemcpy(sv, P.stats, sizeof(sv), hipMemcpyDeviceToHost);
   if (e != hipSuccess) return fail(QSMI_ERR_HIP, std::string("path loop: ") + hipGetErrorString(e));
-  *gaveUp = ctl[1] != 0;
+  *gaveUp = gone != 0;
   *doneOut = done;
   *kernelMs = ms;
   for (int q = 0; q < 4; ++q) stats[q] = (long long)sv[q];
