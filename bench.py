@@ -428,8 +428,9 @@ def main():
     # A = V*S*8 + 2*N*4 (V=2 spectra of S=501*1000 complex64, N=10^6 map
     # floats written and read: a scan by transforms) over its event-timed
     # duration. The data-flow loop (no gather stage of its own) is one kernel,
-    # launched once for 64 waves of nodes; the wave loop's dominant kernel is
-    # the spectrum stage, launched once a wave.
+    # launched for 64 waves of nodes at a time (for fewer where its rate is
+    # judged against the waves': figures per launch are per 64 waves); the wave
+    # loop's dominant kernel is the spectrum stage, launched once a wave.
     V, S, N = 2, (dims[0] // 2 + 1) * dims[1], dims[0] * dims[1]
     a_node = V * S * 8 + 2 * N * 4
     st = stats[-1]

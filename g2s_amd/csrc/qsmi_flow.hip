@@ -1,34 +1,36 @@
 // Data-flow path loop: one persistent kernel simulates the path nodes, every
 // node as soon as its neighbours hold values, without FFTs (gfx950).
 //
-// Schedule. Workgroups take tickets in path order; a ticket is one of G
-// slices (parts of the TI's valid positions) of a node. A node's neighbours
-// precede it on the path, so their tickets were taken before and run on
-// resident workgroups: waiting for their values in the simulation grid (a
+// Schedule. Workgroups take tickets by (dependency level, path index); a
+// ticket is one of G slices (parts of the TI's valid positions) of a node. A
+// node's neighbours are of lower levels, so their tickets were taken before and
+// run on resident workgroups: waiting for their values in the simulation grid (a
 // bounded poll of device-scope atomics) always ends, and there are neither
 // launches nor barriers between dependent nodes. The grid cell itself is the
 // message: a 32-bit word per variable, kPending until the node is written, so
 // nothing else has to be ordered with it. The last slice of a node polls the
 // other slices' K best (64-bit words, all-ones until written), merges, draws
-// and writes.
+// and writes. Levels rather than path indices: the nodes that others wait for
+// come first (151 ms against 182 for 220 x 220 nodes of a 1000 x 1000 image).
 //
 // Scan (k_flow_direct). With x_j the neighbours' values and w_j >= 0 their
 // weights, the map is, up to a constant of the node,
 //     E(p) = -sum_j w_j (x_j - y(p + d_j))^2 - sum_j w_j [class differs],
-// so a partial sum of the cost -E bounds it from below. A wavefront sums 256
-// positions (4 per lane, consecutive in the valid box) over the neighbours,
-// most unusual values first, and drops them together once every partial sum
-// is above the bound: the K-th smallest cost known so far, seeded by the
+// so a partial sum of the cost -E bounds it from below. A wavefront sums two
+// tiles of 16 x 4 positions (2 per lane) over the neighbours, most unusual
+// values first, eight at a time, and drops them together once every partial
+// sum is above the bound: the K-th smallest cost known so far, seeded by the
 // positions the neighbours themselves were copied from. Positions within the
 // bound plus the FP32 error of both sums are kept, and the K best of them are
 // decided in FP64 by the same sum, in the same order, as everywhere else in
 // the library (exact_value in qsmi_band.hip), so the selected positions are
 // those of the exact selection.
-//   Bound by L1 bandwidth: 4 bytes a (position, neighbour) pair against 4 VALU
-//   instructions. A dword a lane runs at 34 TB/s on 256 CUs, 8.5 T pairs/s
-//   (measured; 16-byte loads the same); the valid box is walked as one
-//   sequence, so narrow boxes leave no lane idle. On the 1000 x 1000
-//   log-normal image with n = 80 a node needs 10-40 % of its 80 M pairs.
+//   Bound by issue: a pair is a 4-byte load, two (weights of 1) to four vector
+//   and about one scalar instruction; on the 1000 x 1000 log-normal image with n
+//   = 80 the vector, the scalar and the load unit are each busy for 0.6 of the
+//   time (loads alone: 34 TB/s of L1 on 256 CUs, 8.5 T pairs/s). A node needs
+//   17-30 % of its 80 M pairs there and half of them in white noise, where waves
+//   of transforms are the faster ones: run_flow leaves such paths to them.
 //
 // Scan (k_flow_count). Categorical variables under one kernel weight: E is
 // the weight times the number of agreeing neighbours. The TI is held as one
@@ -36,7 +38,9 @@
 // into bit-sliced counters (carry-save adders of two v_bitop3_b32 each), about
 // 3 instructions a neighbour for 32 positions where the FFT route needs ~8000
 // a position block, and compares them with the K-th count known so far.
-//   Bound by L1 bandwidth too (8 bytes a word, for the funnel shift).
+//   Bound by L1 bandwidth: 16 bytes a load feed three words of 32 positions
+//   (8-byte loads, one word each, run at half the rate: 83 ms against 44 for
+//   the 24 x 24 x 12 part of a 180 x 150 x 120 image).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -63,7 +67,7 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr uint32_t kNoTicket = 0x40000000u;  // above every ticket of a launch (nodes x slices)
 // The word that says so stands in a cache line of its own: waits look at it, and
 // beside the ticket, which every block adds to, that look slowed the tickets
-// (500 x 500, 5 classes and a continuous variable, 60 x 60 nodes: 30 -> 20 ms).
+// (500 x 500, a continuous and a 4-class variable, 60 x 60 nodes: 30 -> 20 ms).
 constexpr int kGaveUp = 64, kCtlWords = 128;
 constexpr unsigned long long kOpen = ~0ull;  // slice result not written yet
 constexpr int kThreads = 256, kWaves = kThreads / 64;
@@ -206,8 +210,9 @@ struct FlowNb {
   float* dt;  // [nVar][n] delta0 terms (direct form)
 };
 
-// A node without neighbours: drawn from the marginal (include/simulation.hpp:
-// 586-606). Thread 0 of the node's last slice.
+// Writes TI position p (kNone: none was valid) into the cell's missing
+// variables, which releases the nodes that wait for them, and into the index
+// image (include/simulation.hpp:658-666). Thread 0 of the node's last slice.
 __device__ void write_cell(FlowArgs& P, unsigned cell, uint32_t p) {
   const long long c = (long long)cell * P.nVar;
   if (p != kNone) st_agent(&P.index[cell], p);
@@ -558,8 +563,11 @@ __device__ __forceinline__ float uniform(float v) {
 // categorical variables. NV: 1 for one variable, else at least their number.
 // COUNT: tiles and steps are counted (a scalar more in the tile loop, 1 % of the
 // scan, so only the segments that are judged by them do).
+// Wavefronts a SIMD: six where the tile loop fits 80 registers, five for the
+// mixed form (two more registers spill into the loop: 543 -> 556 ms on 500 x 500
+// with a continuous and a 4-class variable, 225,000 nodes).
 template <int FORM, int NV, int KT, bool COUNT>
-__global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 && FORM != 2 ? 6 : 5) : 4) k_flow_direct(FlowParams kernArgs) {
+__global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV == 1 ? 6 : 5) : 4) k_flow_direct(FlowParams kernArgs) {
   constexpr bool MIXED = FORM == 2;
   extern __shared__ __align__(16) char dyn[];
   __shared__ FlowShared sh;
@@ -609,6 +617,7 @@ __global__ void __launch_bounds__(kThreads, KT <= 2 ? (NV <= 2 && FORM != 2 ? 6 
       if (cnt == 1)
         for (int v = 0; v < nVar; ++v) given |= !isnan(P.di[(long long)cell * nVar + v]);
       if (!given) {
+        // no neighbour, no value: drawn from the marginal (include/simulation.hpp:586-606)
         if (slice == G - 1 && tid == 0) write_cell(P, cell, (uint32_t)(int)floorf(seed * (float)P.S));
         continue;
       }
@@ -1038,6 +1047,7 @@ __global__ void __launch_bounds__(kThreads) k_flow_count(FlowParams kernArgs) {
       if (cnt == 1)
         for (int v = 0; v < nVar; ++v) given |= !isnan(P.di[(long long)cell * nVar + v]);
       if (!given) {
+        // no neighbour, no value: drawn from the marginal (include/simulation.hpp:586-606)
         if (slice == G - 1 && tid == 0) write_cell(P, cell, (uint32_t)(int)floorf(seed * (float)P.S));
         continue;
       }
@@ -1484,8 +1494,8 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   P.planeWords = rows * P.W0;
   P.zeroPlane = F.nClasses;
   const size_t SD = (size_t)P.sd[0] * P.sd[1] * P.sd[2];
-  // one launch simulates a segment of the path (slots and tickets of its own)
-  // (shorter ones when progress is reported between them)
+  // one launch simulates a segment of the path (slots and tickets of its own),
+  // a shorter one when progress is reported between them
   const size_t seg = std::min<size_t>(std::max<size_t>(nPath, 1),
                                       (size_t)(R.progressSec > 0 ? std::min(F.segment, 8192) : F.segment));
   const size_t slotWords = (size_t)seg * (P.G - 1) * P.K * (F.count ? 1 : 2);

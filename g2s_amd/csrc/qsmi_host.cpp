@@ -847,7 +847,7 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   }
   // dependency levels (1 + the deepest level among a node's path neighbours)
   // on the device; only the levels come back (the data-flow loop waits for
-  // values instead and needs none)
+  // values, but takes its nodes in their order)
   std::vector<int> level(nPath, 0);
   void *dLevel = nullptr, *dLvErr = nullptr;
   if (!rc) rc = dev_upload(nullptr, nPath * sizeof(int), &dLevel);
@@ -880,16 +880,15 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   }
   const auto tNb = clk::now();
   int maxLevel = 0;
-  const size_t nLeveled = level.size();
-  for (size_t i = 0; i < nLeveled; ++i) maxLevel = std::max(maxLevel, level[i]);
+  for (size_t i = 0; i < nPath; ++i) maxLevel = std::max(maxLevel, level[i]);
   // nodes ordered by (level, path order)
   std::vector<size_t> lvStart(maxLevel + 2, 0);
-  for (size_t i = 0; i < nLeveled; ++i) lvStart[level[i] + 1]++;
+  for (size_t i = 0; i < nPath; ++i) lvStart[level[i] + 1]++;
   for (int l = 0; l <= maxLevel; ++l) lvStart[l + 1] += lvStart[l];
-  std::vector<unsigned> order(nLeveled);
+  std::vector<unsigned> order(nPath);
   {
     std::vector<size_t> fillp(lvStart.begin(), lvStart.end() - 1);
-    for (size_t i = 0; i < nLeveled; ++i) order[fillp[level[i]]++] = (unsigned)i;
+    for (size_t i = 0; i < nPath; ++i) order[fillp[level[i]]++] = (unsigned)i;
   }
   // 512 nodes per wave measured best on the 1000x1000 path (fewer launches;
   // 768 no better); the learned proposal keeps its queries in LDS: 256
@@ -1021,7 +1020,7 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
       rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &done, &gaveUp);
       scanned = (long long)nPath;
       waves = (int)R.waveLevel.size();
-      if (!rc && gaveUp) {  // the wave loop, from the start
+      if (!rc && gaveUp) {  // the grid is not usable: the wave loop, from the start
         for (void* p : allocs) (void)hipFree(p);
         qsmi_ti_destroy(ti);
         const double setup = std::chrono::duration<double, std::milli>(t1 - t0).count();

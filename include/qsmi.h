@@ -104,10 +104,17 @@ int qsmi_ti_destroy(qsmi_ti* ti);
  *                 stage timing is not recorded then): 0..1, default 0
  *   "loop.flow"   1: the path loop runs as one persistent kernel that
  *                 simulates every node as soon as its neighbours hold values,
- *                 without transforms, where the request allows it (one TI,
- *                 not circular, no NaN, no learned proposal, record or -nV;
- *                 loop.graph 0), and by waves of transforms from where those
- *                 are the faster: 0..1, default 1; 0: waves from the start
+ *                 without transforms, where the request allows it, and by
+ *                 waves of transforms from where those are the faster: 0..1,
+ *                 default 1; 0: waves from the start. It needs: one TI, not
+ *                 circular, no NaN; no learned proposal, record or -nV; kernel
+ *                 weights in [0, 1e6] and values within 1e12; n x variables <=
+ *                 512, at most 8 variables and 16 one-hot variables, fewer
+ *                 than 2^28 TI values; loop.graph 0. With a continuous
+ *                 variable: tie quantum 0 (the default). Categorical variables
+ *                 only: one kernel weight for all, and a quantum that divides
+ *                 it and is no finer than the default (which a weight of 0.3
+ *                 or a distance kernel does not meet), or quantum 0
  *   "flow.nodes"  path nodes after which that kernel hands over to waves (the
  *                 same bytes): 0..2^30, default 0: where the work that it
  *                 counts says so
