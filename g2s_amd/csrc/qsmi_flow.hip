@@ -1575,7 +1575,7 @@ int run_flow(qsmi_ti* t, const ResidentLoop& R, const FlowPlan& F, double* kerne
   size_t countFrom = judge ? 0 : nPath, verdict = (size_t)std::max(64, R.n);  // nodes counted, then judged
   unsigned long long seen[kFlowStats] = {};
   size_t done = 0, judgedAt = 0;
-  const size_t stop = t->tune.flowNodes > 0 ? std::min(nPath, (size_t)t->tune.flowNodes) : nPath;
+  const size_t stop = t->tune.flowNodes > 0 && !F.alone ? std::min(nPath, (size_t)t->tune.flowNodes) : nPath;
   for (size_t b = 0; b < stop && e == hipSuccess && !slow; b = done) {
     P.node0 = (int)b;
     const bool counted = b >= countFrom;

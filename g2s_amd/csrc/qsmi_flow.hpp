@@ -19,6 +19,7 @@ struct FlowPlan {
   float rare[kFlowMaxCat] = {};                // per class: 1 - its share of the TI
   int inFlight = 1 << 20;  // path nodes simulated at the same time, at most
   int segment = 65536;     // path nodes per launch
+  bool alone = false;      // the whole path, whatever the waves would take
   // what the wave loop takes, microseconds: a wave, a node, its spectra and
   // buffers (waveNodeUs 0: the path is never handed over to it)
   double waveUs = 0.0, waveNodeUs = 0.0, waveSetupUs = 0.0;

@@ -37,7 +37,10 @@ namespace {
 
 int hfail(int code, const std::string& m) { return qsmi_internal_fail(code, m.c_str()); }
 
-int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow);
+// the path loops that a run may take
+enum class Loops { both, waves, flow };
+
+int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, Loops loops);
 
 struct KernelImg {
   int D = 0;
@@ -365,7 +368,7 @@ int qsmi_path(size_t cells, const unsigned char* informed, unsigned seed, unsign
 // ---------------------------------------------------------------------------
 // In-memory QS run
 // ---------------------------------------------------------------------------
-int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) { return qs_run(rq, rs, true); }
+int qsmi_qs_run_in_memory(const qsmi_qs_request* rq, qsmi_qs_result* rs) { return qs_run(rq, rs, Loops::both); }
 
 }  // extern "C"
 
@@ -469,7 +472,7 @@ void wave_cost(const qsmi_ti* ti, int V, int n, int K, qsmi::FlowPlan* F) {
   F->waveSetupUs = 1000.0 + 0.0065 * V * (double)ti->S;
 }
 
-int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
+int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, Loops loops) {
   using clk = std::chrono::steady_clock;
   if (!rq || !rs || !rs->simulation || !rs->index) return hfail(QSMI_ERR_ARG, "null argument");
   const int D = rq->ndim;
@@ -702,7 +705,7 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
   qsmi_ti* ti = nullptr;
   qsmi_device* dev = nullptr;
   qsmi::FlowPlan flow;
-  bool useFlow = allowFlow && !cross &&
+  bool useFlow = loops != Loops::waves && !cross &&
                  plan_flow(rq, qsmi::default_tune(), D, tiIn, S, SD, nMax, ncat, catvals, ker.data, nExp, quantum,
                            defaultQuantum, &flow);
   int rc = QSMI_OK;
@@ -1014,25 +1017,30 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
         flow.inFlight = rq->waveSize;
         flow.segment = (int)std::min<long long>(flow.segment, 64ll * rq->waveSize);
       }
-      if (!flow.count) wave_cost(ti, nSub, nMax, (int)std::ceil(kMax), &flow);
+      flow.alone = loops == Loops::flow;
+      if (!flow.count && !flow.alone) wave_cost(ti, nSub, nMax, (int)std::ceil(kMax), &flow);
       size_t done = 0;
       bool gaveUp = false;
       rc = qsmi::run_flow(ti, R, flow, &stageMs[0], bandStats, &done, &gaveUp);
       scanned = (long long)nPath;
       waves = (int)R.waveLevel.size();
-      if (!rc && gaveUp) {  // the grid is not usable: the wave loop, from the start
+      // the run again from its start, by the other loop; what this attempt took counts
+      auto again = [&](Loops other) -> int {
         for (void* p : allocs) (void)hipFree(p);
+        if (dev) qsmi_device_destroy(dev);
         qsmi_ti_destroy(ti);
+        (void)hipGetLastError();
         const double setup = std::chrono::duration<double, std::milli>(t1 - t0).count();
         const double lost = std::chrono::duration<double, std::milli>(clk::now() - t1).count();
-        rc = qs_run(rq, rs, false);
-        if (!rc) {  // what the first attempt took counts
+        const int r = qs_run(rq, rs, other);
+        if (!r) {
           rs->setupMs += setup;
           rs->pathLoopMs += lost;
           rs->phaseMs[3] += lost;
         }
-        return rc;
-      }
+        return r;
+      };
+      if (!rc && gaveUp) return again(Loops::waves);  // the grid is not usable
       if (!rc && done < nPath) {  // the rest by waves
         qsmi_ti_destroy(ti);
         ti = nullptr;
@@ -1053,6 +1061,7 @@ int qs_run(const qsmi_qs_request* rq, qsmi_qs_result* rs, bool allowFlow) {
             bandStats[q] += band[q];
           }
         }
+        if (rc) return again(Loops::flow);  // no memory for the spectra or the waves
       }
     } else {
       rc = qsmi::run_resident_waves(dev, R, stageMs, &scanned, &waves, bandStats);

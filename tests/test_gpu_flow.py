@@ -146,6 +146,24 @@ def test_flow_without_valid_position(kind):
     assert 0 < empty < di.size
 
 
+def test_flow_without_memory_for_waves():
+    """A hand-over to waves that do not fit (levels of 100,000 nodes of a 1000
+    x 1000 image, 8 MB each): the data-flow loop simulates the whole path."""
+    rng = np.random.default_rng(19)
+    dims, sdims = (1000, 1000), (1000, 1000)
+    args = (_field(dims, rng, "cont").astype(np.float32), dims, np.full(sdims[0] * sdims[1], np.nan, np.float32),
+            sdims, [0], 2, 1.0, 3)
+    out = []
+    try:
+        for nodes in (0, 1000):
+            g2s_amd.set_default_tuning("flow.nodes", nodes)
+            out.append(g2s_amd.qs(*args, wave_size=1 << 20, stage_timing=True))
+    finally:
+        g2s_amd.set_default_tuning("flow.nodes", 0)
+    assert out[0][0].tobytes() == out[1][0].tobytes() and out[0][1].tobytes() == out[1][1].tobytes()
+    assert out[0][2]["gather_ms"] == out[1][2]["gather_ms"] == 0.0
+
+
 def test_flow_slices_and_segments():
     """An image large enough for several slices a node and a path of several
     launches (64 nodes in flight, 64 x 64 a launch)."""
