@@ -6,6 +6,8 @@ import os
 import shutil
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -22,15 +24,13 @@ FLAGS = [
     "-std=c++17",
     "--offload-arch=gfx950",
     "-fPIC",
-    "-shared",
     # no packed FP32 instructions in device code
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
     "-Wno-unused-value",
     "-I" + os.path.join(ROOT, "include"),
-    "-lpthread",
-    "-lz",
 ]
+LINK = ["-shared", "-lpthread", "-lz"]
 
 
 def hipcc():
@@ -40,17 +40,24 @@ def hipcc():
     raise RuntimeError("hipcc not found: the qsmi library cannot be built")
 
 
-def build(verbose=False):
-    """Compile every source into g2s_amd/libqsmi.so (always recompiles)."""
-    srcs = [os.path.join(CSRC, s) for s in SOURCES]
-    tmp = LIB + ".tmp"
-    cmd = [hipcc()] + FLAGS + ["-o", tmp] + srcs
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         sys.stderr.write(r.stdout + r.stderr)
         raise RuntimeError("hipcc failed building libqsmi.so")
+
+
+def build(verbose=False):
+    """Compile every source into g2s_amd/libqsmi.so (always recompiles), the
+    sources side by side."""
+    tmp = LIB + ".tmp"
+    with tempfile.TemporaryDirectory() as objs, ThreadPoolExecutor(8) as pool:
+        out = [os.path.join(objs, s + ".o") for s in SOURCES]
+        cmds = [[hipcc()] + FLAGS + ["-c", "-o", o, os.path.join(CSRC, s)] for s, o in zip(SOURCES, out)]
+        list(pool.map(lambda c: _run(c, verbose), cmds))
+        _run([hipcc()] + FLAGS + ["-o", tmp] + out + LINK, verbose)
     os.replace(tmp, LIB)
     return LIB
 
